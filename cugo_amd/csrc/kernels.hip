@@ -113,6 +113,15 @@ __device__ inline void stage_out(const u64* lds, u64* dst, const i64* ids_lds, i
   }
 }
 
+// The row at `row` (in LDS or global memory) unpacked again, for torch_step's reload: the
+// offset is opaque, so the compiler reads the row anew where it is needed (only where an
+// action failed) instead of keeping the first read's ~75 registers.
+template <class P>
+__device__ inline Env reread_row(const P* rows, i32 word) {
+  asm volatile("" : "+v"(word));
+  return unpack_row(rows + word);
+}
+
 __device__ inline u16 clamp_action(i64 raw) {  // torch50_ext.cu:96-99
   return raw >= 0 && raw < kActionCount ? (u16)raw : kInvalidAction16;
 }
@@ -333,6 +342,23 @@ __device__ inline u64 sampler_seed(u64 seed) {
   return v != 0 ? v : 1ull;
 }
 
+// v % t for 1 <= t < 256, 16 bits of v at a time: r < t, so r * 65,536 + the next 16 bits is
+// below 2^24 and exact in a float, its quotient by t is below 65,536, and the rounded
+// product with the approximate reciprocal is off by less than one, so one correction
+// each way makes it exact.  (A 64-bit integer remainder compiles to ~130 instructions.)
+__device__ inline u32 mod_small(u64 v, u32 t) {
+  const float inv = __builtin_amdgcn_rcpf((float)t);
+  u32 r = 0;
+#pragma unroll
+  for (int k = 3; k >= 0; --k) {
+    const u32 x = (r << 16) | (u32)((v >> (16 * k)) & 0xFFFFu);
+    const u32 q = (u32)((float)x * inv);
+    const i32 d = (i32)(x - q * t);
+    r = (u32)(d < 0 ? d + (i32)t : d >= (i32)t ? d - (i32)t : d);
+  }
+  return r;
+}
+
 // Uniform draw over the set bits of a 179-bit action mask (actions 0..63 in m0, 64..127
 // in m1, 128..178 in m2): one xorshift64 step of the sampler word x, then the
 // (value % count)-th set bit.  -1, with x untouched, when no bit is set.
@@ -340,10 +366,13 @@ __device__ inline i64 draw_legal(u64 m0, u64 m1, u64 m2, u64& x) {
   const u32 c0 = popc(m0), c1 = popc(m1);
   const u32 total = c0 + c1 + popc(m2);
   if (total == 0) return -1;
-  const u32 pick = (u32)(xorshift64(x) % total);
-  if (pick < c0) return select_rank(m0, pick);
-  if (pick < c0 + c1) return 64 + select_rank(m1, pick - c0);
-  return 128 + select_rank(m2, pick - c0 - c1);
+  u32 pick = mod_small(xorshift64(x), total);
+  // one rank select on the word that holds the pick (the three words' selects in branches
+  // would each run in a wave whose picks fall in all of them)
+  const bool past0 = pick >= c0, past1 = pick >= c0 + c1;
+  const u64 word = past1 ? m2 : past0 ? m1 : m0;
+  pick -= past1 ? c0 + c1 : past0 ? c0 : 0u;
+  return (past1 ? 128 : past0 ? 64 : 0) + (i64)select_rank_in(word, pick);
 }
 
 // kSample: also draw each row's random-policy action from its legal mask while the mask
@@ -477,7 +506,8 @@ __global__ __launch_bounds__(kStepThreads) void step_kernel(u64* states, i64 env
     i64* evr = ev + lane * kEventWords;
     if (ok) {
       Env e = unpack_row(row);
-      const StepOut so = torch_step(e, clamp_action(actions[i]));
+      const StepOut so = torch_step(e, clamp_action(actions[i]),
+                                    [&] { return reread_row(rows, lane * kRowWords); });
       if (kEvents) {
         if (so.committed) {
           // make_torch_event50 against the untouched row still in LDS
@@ -576,7 +606,8 @@ __global__ __launch_bounds__(kTile) void branch_kernel(const u64* parents, i64 e
 #pragma unroll
       for (int k = 0; k < kRowWords; ++k) row[k] = src[k];
       Env e = unpack_row(row);
-      const StepOut so = torch_step(e, clamp_action(actions[i]));
+      const StepOut so = torch_step(e, clamp_action(actions[i]),
+                                    [&] { return reread_row(src, 0); });
       pack_row(e, row);
       reward[i] = (float)so.reward0;
       done[i] = so.done;
@@ -681,7 +712,7 @@ void play_kernel(
         // packet from the very Env that is then stepped leaves an engine temporary in
         // private memory.
         Env g = e;
-        const StepOut so = torch_step_head(g, clamp_action(a), head);
+        const StepOut so = torch_step_head(g, clamp_action(a), head, [&] { return e; });
         const i64 at = i + (i64)(s - 1) * step_rows;  // step s - 1's output row
         reward[at] = (float)so.reward0;
         done[at] = so.done;
@@ -779,7 +810,8 @@ void step_observe_kernel(u64* states, i64 n, const i64* actions, float* reward, 
     const u32 sgen = ar.spare_gen[srow];  // issued before the step so its latency hides
     u64* row = rows + lane * kRowWords;
     Env e = unpack_row(row);
-    const StepOut so = torch_step(e, clamp_action(actions[i]));
+    const StepOut so = torch_step(e, clamp_action(actions[i]),
+                                  [&] { return reread_row(rows, lane * kRowWords); });
     reward[i] = (float)so.reward0;
     done[i] = so.done;
     nagari[i] = so.nagari;
@@ -848,7 +880,8 @@ __global__ __launch_bounds__(kPlayThreads) void branch_observe_kernel(
   if (active) {
     e = unpack_row(t.rows + lane * kRowWords);
     if (valid_id(tile_ids[lane], env_count)) {
-      const StepOut so = torch_step(e, clamp_action(actions[i]));
+      const StepOut so = torch_step(e, clamp_action(actions[i]),
+                                    [&] { return reread_row(t.rows, lane * kRowWords); });
       reward[i] = (float)so.reward0;
       done[i] = so.done;
       nagari[i] = so.nagari;
