@@ -573,41 +573,47 @@ __global__ __launch_bounds__(kStepThreads) void step_kernel(u64* states, i64 env
 // branch_indexed (torch50_ext.cu:288-314): each lane reads its parent row straight from
 // global memory (branching children of one root read the same row, so a wave's loads are
 // broadcasts from L2), steps it in registers, and the wave's 64 child rows go out through
-// LDS as one contiguous block.  The transition holds ~200 VGPRs, which allows two waves
-// per SIMD; capping registers for three or four waves spills 144 / 356 bytes a lane and
-// measured 1.35x / 2.7x slower on 1,048,576 children, and staging the parents through LDS
-// as well, as the other step kernels do, measured 1.13x slower.
-// kRows children a wavefront: at 1,048,576 children (16,384 wavefronts, many rounds) 64
-// took 0.103 ms, 48 0.126 and 32 0.153: fewer children a wavefront run fewer divergent
-// rule paths each, but the launch issues more wavefronts of the same length.
-// Waves whose 64 children share one parent (C3's layout) were also given a path that
+// LDS as contiguous blocks.  An action that fails reads its parent again, so the
+// transition keeps one state in registers: 168 VGPRs, three waves per SIMD (with a second
+// state kept they were 198 and two waves; 262,144 children 31.7 -> 27.4 us).  Capping
+// registers for four waves spills ~150 bytes a lane; staging the parents through LDS as
+// well, as the other step kernels do, measured 1.13x slower when two waves fit.
+// kRows children a wavefront: see branch_rows().
+// Waves whose 64 children share one parent were also given a path that
 // reads the parent with scalar loads and builds its legality head once in scalar
 // registers: VALU instructions fell from 2,095 to 1,978 a wave (the head is that
-// small a part of the step), SALU rose from 634 to 871, VGPRs stayed at 198, and the
-// launch took the same time (0.100-0.102 ms against 0.099-0.105), so it was dropped.
+// small a part of the step), SALU rose from 634 to 871, and the launch took the same time
+// (0.100-0.102 ms against 0.099-0.105), so it was dropped.
 // Tiles of 256 children grouped by action in LDS before the step (a counting sort, so a
 // wavefront's lanes share one or two actions' rule paths) took 0.110 ms: dropped too.
 template <int kRows>
-__global__ __launch_bounds__(kTile) void branch_kernel(const u64* parents, i64 env_count,
+__global__ __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(3))) void branch_kernel(const u64* parents, i64 env_count,
                                                        const i64* ids, const i64* actions,
                                                        i64 n, u64* children, float* reward,
                                                        u8* done, u8* nagari, i16* status,
                                                        u8* committed) {
-  __shared__ u64 tile[kRows * kRowWords];
+  constexpr int kStage = kRows < 32 ? kRows : 32;  // child rows staged at a time
+  __shared__ u64 tile[kStage * kRowWords];
   const int lane = threadIdx.x;
   const i64 base = (i64)blockIdx.x * kRows;
   const i64 i = base + lane;
   const int count = n - base < kRows ? (int)(n - base) : kRows;
+  u64 row[kRowWords];
   if (lane < kRows && i < n) {
     const i64 id = ids[i];
-    u64 row[kRowWords];
     if (valid_id(id, env_count)) {
-      const u64* src = parents + id * kRowWords;
+      // one register (a batch of 2^32 rows, 1 TB, is past the memory)
+      const u32 parent = (u32)id;
+      const u64* src = parents + (u64)parent * kRowWords;
 #pragma unroll
       for (int k = 0; k < kRowWords; ++k) row[k] = src[k];
       Env e = unpack_row(row);
       const StepOut so = torch_step(e, clamp_action(actions[i]),
-                                    [&] { return reread_row(src, 0); });
+                                    [&] {
+                                      u32 again = parent;  // see reread_row
+                                      asm volatile("" : "+v"(again));
+                                      return unpack_row(parents + (u64)again * kRowWords);
+                                    });
       pack_row(e, row);
       reward[i] = (float)so.reward0;
       done[i] = so.done;
@@ -623,19 +629,28 @@ __global__ __launch_bounds__(kTile) void branch_kernel(const u64* parents, i64 e
       status[i] = CUGO_INVALID_INDEX_STATUS;
       committed[i] = 0;
     }
-#pragma unroll
-    for (int k = 0; k < kRowWords; ++k) tile[lane * kRowWords + k] = row[k];
   }
-  // The tile's child rows leave as one contiguous block: stored from registers, a store
-  // instruction wrote 8 bytes into each of 64 rows 248 bytes apart, and the L1's queue of
-  // partial-line writes stalled the wave most of the time.
-  __syncthreads();
-  u64* out = children + base * kRowWords;
-  const int words = count * kRowWords;
+  // The tile's child rows leave as contiguous blocks of kStage rows through LDS: stored from
+  // registers, a store instruction wrote 8 bytes into each of 64 rows 248 bytes apart, and
+  // the L1's queue of partial-line writes stalled the wave most of the time.  Half a tile at
+  // a time, so that the LDS holds the wavefronts that the registers allow.
 #pragma unroll
-  for (int j = 0; j < (kRows * kRowWords + kTile - 1) / kTile; ++j) {
-    const int w = j * kTile + lane;
-    if (w < words) out[w] = tile[w];
+  for (int h = 0; h < kRows; h += kStage) {
+    if (h >= count) break;
+    if (h > 0) __syncthreads();
+    if (lane >= h && lane < h + kStage && lane < count) {
+#pragma unroll
+      for (int k = 0; k < kRowWords; ++k) tile[(lane - h) * kRowWords + k] = row[k];
+    }
+    __syncthreads();
+    u64* out = children + (base + h) * kRowWords;
+    const int left = count - h;
+    const int words = (left < kStage ? left : kStage) * kRowWords;
+#pragma unroll
+    for (int j = 0; j < (kStage * kRowWords + kTile - 1) / kTile; ++j) {
+      const int w = j * kTile + lane;
+      if (w < words) out[w] = tile[w];
+    }
   }
 }
 
@@ -775,6 +790,145 @@ void play_kernel(
   }
 }
 
+// The same steps for batches that leave SIMDs without a computing wave at 64 games a tile
+// (see play_rows): tiles of kRows games, two waves each, each wave with a part of the step
+// that the other does not wait for:
+//   * wave 0 plays: it keeps the games in registers for the whole launch and runs the
+//     chain step -> (next game) -> legal mask -> draw, which is all that the next step
+//     depends on, and leaves each state's row in LDS;
+//   * wave 1 observes: it unpacks that row, builds the observation's records and stores
+//     them, one step behind (wave 0 takes over what is left of larger tiles' stores).
+// So the latency of a step is the longer of the two parts instead of their sum: 3,001 games
+// on 4-game tiles 413 -> 318 us a 32-step launch.  One barrier a step hands a state over;
+// wave 0 overwrites the row in LDS only once wave 1 has counted it as unpacked (`seen`;
+// wave 1 unpacks first thing after the barrier, so wave 0 does not wait in practice).  An
+// action that fails reads its state again from that row.  At 65,536 games, where the
+// stores bound the launch, play_kernel is the better one (1,030 against 1,049 us): its
+// wave 1 stores from the first instruction of a step on.
+template <int kRows>
+__global__ __launch_bounds__(kPlayThreads) __attribute__((amdgpu_waves_per_eu(2)))
+void play_split_kernel(
+    u64* states, i64 n, u64* sampler, float* features, u8* legal, u8* player, u8* obs_done,
+    i16* obs_status, i64* actions, float* reward, u8* done, u8* nagari, i16* status,
+    u8* committed, AutoReset ar, int steps, i64 step_rows) {
+  static_assert(kRows >= 4 && kRows % 4 == 0 && kRows <= kTile, "mask rows in whole dwords");
+  constexpr bool kJoin = kRows >= 16;  // wave 0 joins the stores
+  __shared__ u64 rows[kRows * kRowWords];  // the games in the state being observed
+  __shared__ RecordBufferOf<kRows> rb;     // wave 1's: that state's observation
+  __shared__ int next_item;                // wave 1's: store_observation's work counter
+  __shared__ int seen;                     // states that wave 1 has unpacked
+  __shared__ int ready;                    // states whose records it has built
+  const i64 base = (i64)blockIdx.x * kRows;
+  const int count = n - base < kRows ? (int)(n - base) : kRows;
+  const int tid = threadIdx.x;
+  const int lane = tid & (kTile - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kTile);
+  const i64 i = base + lane;
+  if (tid == 0) seen = ready = 0;
+  {
+    const u64* src = states + base * kRowWords;
+    for (int j = tid; j < count * kRowWords; j += kPlayThreads) rows[j] = src[j];
+  }
+  __syncthreads();
+  const bool active = lane < count;
+  if (wave == 0) {
+    u32 gen = 0;
+    u32 have = 0;  // bit k: the spare of generation gen + 1 + k is pre-dealt
+    u64 xc = 0;    // the committed sampler state
+    u64 xt = 0;    // the sampler state after the draw (committed with the step)
+    i64 a = -1;
+    Env e;  // the game this lane plays (its next game once it finishes)
+    PacketHead head{};
+    if (active) {
+      gen = ar.generation[i];
+      for (u32 k = 0; k <= ar.slot_mask; ++k)
+        if (ar.spare_gen[spare_row(ar, i, gen + 1u + k)] == gen + 1u + k) have |= 1u << k;
+      xc = sampler[i];
+      e = unpack_row(rows + lane * kRowWords);
+    }
+    for (int s = 0; s < steps; ++s) {
+      if (active) {
+        head = packet_head(e);
+        xt = xc;
+        a = draw_legal(head.legal.w0, head.legal.w1, head.legal.w2, xt);
+        const i64 at = i + (i64)s * step_rows;  // step s's output row
+        actions[at] = a;
+        const StepOut so = torch_step_head(
+            e, clamp_action(a), head, [&] { return reread_row(rows, lane * kRowWords); });
+        reward[at] = (float)so.reward0;
+        done[at] = so.done;
+        nagari[at] = so.nagari;
+        status[at] = (i16)so.status;
+        committed[at] = so.committed;
+        if (so.done) {  // the next game: this generation's spare, or dealt here if stale
+          ++gen;
+          const u64 seed = ar.base_seed + (u64)i + ar.stride * gen;
+          xc = sampler_seed(seed);
+          // A stale spare gets its game dealt into its own slot first (out of line: the
+          // deal inlined here doubles the loop's register pressure for a rare path).
+          const i64 row = spare_row(ar, i, gen);
+          if ((have & 1u) == 0) deal_into(seed, (u32)(i & 1), ar.spares + row * kRowWords);
+          e = unpack_row(ar.spares + row * kRowWords);
+          have >>= 1;
+        } else if (a >= 0) {
+          xc = xt;
+        }
+      }
+      while (__hip_atomic_load(&seen, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) <= s)
+        __builtin_amdgcn_s_sleep(1);
+      if (active) pack_row(e, rows + lane * kRowWords);
+      // take over what is left of the state's stores, if its records are there
+      if (kJoin &&
+          __hip_atomic_load(&ready, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) > s)
+        store_observation<kPlayClaim, false, kRows>(
+            rb, base, count, features + (i64)s * step_rows * kFeatureCount,
+            legal + (i64)s * step_rows * kActionCount, &next_item);
+      __syncthreads();
+    }
+    if (active) {
+      ar.generation[i] = gen;
+      sampler[i] = xc;
+    }
+  } else {
+    for (int s = 0; s < steps; ++s) {
+      Env e;
+      if (active) e = unpack_row(rows + lane * kRowWords);
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+      if (lane == 0) {
+        next_item = 0;
+        __hip_atomic_store(&seen, s + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+      }
+      const i64 before = (i64)s * step_rows;  // the rows of the steps before
+      if (active) {
+        const Packet pk = make_packet(e);
+        FeatRow fr;
+        feature_row(pk, c_stop_bits, fr);
+        feature_record(fr, rb.rec[lane]);
+        rb.legal[lane][0] = pk.head.legal.w0;
+        rb.legal[lane][1] = pk.head.legal.w1;
+        rb.legal[lane][2] = pk.head.legal.w2;
+        player[i + before] = pk.head.player;
+        obs_done[i + before] = e.done != 0;
+        obs_status[i + before] = (i16)pk.head.status;
+      }
+      // the records pass between the lanes of this wave, and to wave 0 where it joins
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+      if (kJoin && lane == 0)
+        __hip_atomic_store(&ready, s + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+      store_observation<kPlayClaim, false, kRows>(rb, base, count,
+                                                  features + before * kFeatureCount,
+                                                  legal + before * kActionCount, &next_item);
+      __syncthreads();
+    }
+  }
+  {
+    u64* out = states + base * kRowWords;
+    for (int j = tid; j < count * kRowWords; j += kPlayThreads) out[j] = rows[j];
+  }
+}
+
 // ------------------------------------------------------------ step + observe ----
 // step_kernel<3> (step with the caller's actions, then the auto-reset of finished rows)
 // followed by observe_kernel of the new states, in one launch: the PPO rollout's engine
@@ -784,8 +938,6 @@ void play_kernel(
 // observation records in LDS and packs the rows; then both waves store the observation
 // and the rows.  The rows are read and written once, where the two launches read them
 // twice and wrote them once more.
-constexpr int kStepObserveRows = 32;  // games a tile (see cugo_step_observe_spares)
-
 template <bool kBf16, int kRows, int kThreads>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
 void step_observe_kernel(u64* states, i64 n, const i64* actions, float* reward, u8* done,
@@ -825,6 +977,7 @@ void step_observe_kernel(u64* states, i64 n, const i64* actions, float* reward, 
       if (sgen != gen) deal_into(seed, (u32)(i & 1), ar.spares + srow * kRowWords);
       e = unpack_row(ar.spares + srow * kRowWords);
     }
+    pack_row(e, row);  // before the observation, which then need not keep all of e
     const Packet pk = make_packet(e);
     FeatRow fr;
     feature_row(pk, c_stop_bits, fr);
@@ -835,7 +988,6 @@ void step_observe_kernel(u64* states, i64 n, const i64* actions, float* reward, 
     player[i] = pk.head.player;
     obs_done[i] = e.done != 0;
     obs_status[i] = (i16)pk.head.status;
-    pack_row(e, row);
   }
   __syncthreads();
   store_observation<kPlayClaim, kBf16, kRows>(rb, base, count, features, legal, &next_item);
@@ -845,19 +997,20 @@ void step_observe_kernel(u64* states, i64 n, const i64* actions, float* reward, 
 // ---------------------------------------------------------- branch + observe ----
 // branch_indexed then observe_indexed of the children (the reference's callers do exactly
 // this, python/cugo_ppo50.py:96-98), in one launch with the same outputs.  Two waves per
-// tile of 64 children: wave 0 gathers the parents, steps the clones and builds the
+// tile of kRows children: wave 0 gathers the parents, steps the clones and builds the
 // children's observation records in LDS; then wave 1 stores the observations while wave 0
 // writes the child rows from registers (each lane its own row), so the children are never
 // read back, and joins the stores after.
+template <int kRows>
 __global__ __launch_bounds__(kPlayThreads) void branch_observe_kernel(
     const u64* parents, i64 env_count, const i64* ids, const i64* actions, i64 n,
     u64* children, float* reward, u8* done, u8* nagari, i16* status, u8* committed,
     float* features, u8* legal, u8* player, u8* obs_done, i16* obs_status) {
-  __shared__ ObserveTile t;
-  __shared__ i64 tile_ids[kTile];
+  __shared__ ObserveTileOf<kRows> t;
+  __shared__ i64 tile_ids[kRows];
   __shared__ int next_item;  // store_observation's work counter
-  const i64 base = tile_base();
-  const int count = tile_count(base, n);
+  const i64 base = (i64)blockIdx.x * kRows;
+  const int count = n - base < kRows ? (int)(n - base) : kRows;
   const int tid = threadIdx.x;
   const int lane = tid & (kTile - 1);
   const int wave = tid / kTile;
@@ -919,9 +1072,11 @@ __global__ __launch_bounds__(kPlayThreads) void branch_observe_kernel(
       for (int k = 0; k < kRowWords; ++k) out[k] = row[k];
     }
   }
-  // (Staging these rows through LDS as branch_kernel does measured 5 % slower here: wave
-  // 0 joins the observation's stores later.)
-  store_observation<2>(t.out, base, count, features, legal, &next_item);  // wave 0 after its rows
+  // Keeping the child in registers through the observation costs the third wave a SIMD (204
+  // VGPRs against 173), but the rows written before it are slower where the output passes
+  // the last-level cache: 1,048,576 children 670 us so, 737 with the rows from registers
+  // right after the step, 698 with wave 1 copying them from LDS beside the observation.
+  store_observation<2, false, kRows>(t.out, base, count, features, legal, &next_item);  // wave 0 after its rows
 }
 
 // ----------------------------------------------------------- calibration ----
@@ -1228,11 +1383,12 @@ __global__ __launch_bounds__(256) void accept_worlds_kernel(
 // instruction issue; one wave per workgroup lets a wave whose games end early retire.
 constexpr int kCanonicalWords = 5;
 
+template <int kRows>
 __global__ __launch_bounds__(kTile) void canonical_kernel(const i64* seeds, const i64* first,
                                                           i64 n, u32 max_actions, i64* out) {
-  __shared__ i64 digest[kTile * kCanonicalWords];
-  const i64 base = tile_base();
-  const int count = tile_count(base, n);
+  __shared__ i64 digest[kRows * kCanonicalWords];
+  const i64 base = (i64)blockIdx.x * kRows;
+  const int count = n - base < kRows ? (int)(n - base) : kRows;
   const int lane = threadIdx.x;
   if (lane < count) {
     Env e = create_env((u64)seeds[base + lane], (u32)(first[base + lane] & 1));
@@ -1292,22 +1448,69 @@ inline int device_cus() {
   return cached[dev];
 }
 
-// step_kernel launch: two waves per tile while all tiles fit at once (four per CU).
-// Games a tile of the observe and step kernels, by batch.  A wavefront runs the union of
-// its games' rule paths, so at small batches (every tile resident, most SIMDs without a
-// computing wavefront) smaller tiles finish sooner; at large ones the wavefronts of
-// 64 games issue fewer instructions in all.  Measured on MI355X (us a launch for 64 / 32 /
-// 16 games a tile, graphs of 20 launches on mid-game rows):
-//   observe            n = 4,096: 20.6 / 15.7 / 12.4    16,384: 22.8 / 18.8 / 16.5
-//                      32,768: 28.5 / 24.9 / 31.5       65,536: 41.5 / 46.5 / 50.2
-//   step_events_indexed 2,048: 19.3 / 18.7 / 14.5       8,192: 20.0 / 18.9 / 19.9
-//                      32,768: 24.5 / 21.5 / 22.6       65,536: 26.6 / 47.8 / 41.0
-inline int obs_rows(int64_t n) { return n <= 16384 ? 16 : n <= 32768 ? 32 : kTile; }
-inline int step_rows(int64_t n) { return n <= 4096 ? 16 : n <= 32768 ? 32 : kTile; }
+// Games a tile, by batch.  A wavefront runs the union of its games' rule paths, one after
+// the other, so while most SIMDs have no computing wavefront the tile with the fewest games
+// finishes first; once every SIMD has one or two, fewer games a tile only add wavefronts
+// that wait for a SIMD.  The lines lie where a grid passes one or two wavefronts a SIMD
+// (1,024 SIMDs).  Measured on MI355X, us a call (64 / 32 / 16 / 8 / 4 games a tile, graphs
+// or bursts of launches on mid-game rows; the start of a launch is ~3 us of each):
+//   play_random x 32    n = 3,001: 828 / 548 / 408 / 386 / 321     8,192: 808 / 552 / 460 / 374
+//                       16,384: 819 / 612 / 485                    32,768: 900 / 661
+//   observe             700: 19.6 / 14.3 / 11.4 / 9.6 / 8.5        4,096: 20.6 / 15.5 / 12.5 / 12.1 / 11.7
+//                       8,192: 21.4 / 15.9 / 14.7 / 13.6 / 20.4    16,384: 22.4 / 18.3 / 15.8 / 24.8
+//                       32,768: 28.3 / 24.6 / 30.7                 65,536: 41.1 / 44.8 / 49.0
+//   step                700: 15.3 / 14.1 / 12.4 / 11.2 / 10.3      2,048: 16.1 / 15.4 / 13.5 / 12.5 / 13.7
+//                       4,096: 15.9 / 15.3 / 14.6 / 14.8 / 18.1    8,192: 16.1 / 16.0 / 18.0 / 19.5 / 13.5
+//                       16,384: 17.6 / 16.4 / 15.9 / 16.2 / 23.6   65,536: 23.2 / 39.7 / 34.9
+//   step_observe, with the sampler before it
+//                       1,024: 48.2 / 40.0 / 34.1 / 31.3 / 27.1    8,192: 50.8 / 42.9 / 41.1 / 40.3 / 34.1
+//                       16,384: 55.1 / 47.5 / 42.5 / 42.8 / -      32,768: 64.7 / 55.4 / 81.0
+//                       65,536: 77.9 / 110.8
+//   branch              2,500: 12.5 / 11.5 / 11.0 / 12.1           20,000: 13.1 / 12.0 / 12.5 / 14.9
+//                       60,000: 14.9 / 15.1 / 20.8
+//   branch_observe (64 / 32 / 16 / 4)
+//                       2,000: 33.2 / 24.8 / 21.0 / 19.9           4,096: 33.2 / 25.6 / 21.6 / 22.0
+//                       16,384: 35.9 / 28.8 / 23.8 / 61.5          32,768: 41.7 / 33.4 / 48.0
+//                       65,536: 54.6 / 67.4 / 78.0
+//   rollout_canonical (64 / 32 / 16 / 8 / 4 / 2 / 1)
+//                       256: 250 / 252 / 231 / 209 / 196 / 177 / 152
+//                       1,024: 260 / 267 / 241 / 216 / 195 / 250 / 305
+//                       4,096: 259 / 284 / 251 / 294 / 392         32,768: 278 / 246 / 287
+// Grids of one-wavefront workgroups between one and about five a CU run slower than smaller
+// and larger ones (the same loop of plain FMAs takes 11 % longer at 512 wavefronts than
+// at 256 or 1,024), which is why the step's line for 4,096 rows is 16 games and the one
+// for 8,192 is 4.
+inline int play_rows(int64_t n) {
+  return n <= 4096 ? 4 : n <= 8192 ? 8 : n <= 16384 ? 16 : n <= 32768 ? 32 : kTile;
+}
+inline int obs_rows(int64_t n) { return play_rows(n); }
+inline int step_rows(int64_t n) {
+  if (n <= 4096) return n <= 1024 ? 4 : n <= 2048 ? 8 : 16;
+  return n <= 8192 ? 4 : n <= 16384 ? 16 : n <= 32768 ? 32 : kTile;
+}
+inline int step_observe_rows(int64_t n) {
+  return n <= 8192 ? 4 : n <= 16384 ? 16 : n <= 32768 ? 32 : kTile;
+}
+inline int branch_rows(int64_t n) { return n <= 4096 ? 16 : n <= 32768 ? 32 : kTile; }
+inline int branch_observe_rows(int64_t n) {
+  return n <= 2048 ? 4 : n <= 16384 ? 16 : n <= 32768 ? 32 : kTile;
+}
+inline int canonical_rows(int64_t n) {
+  if (n <= 4096) return n <= 256 ? 1 : n <= 512 ? 2 : n <= 1024 ? 4 : n <= 2048 ? 8 : 16;
+  return n > 16384 && n <= 32768 ? 32 : kTile;
+}
 
 template <bool kIndexed, bool kSample, bool kBf16, class... Args>
 inline void launch_observe(int64_t n, hipStream_t stream, Args... args) {
   switch (obs_rows(n)) {
+    case 4:
+      observe_kernel<kIndexed, kSample, kBf16, 4>
+          <<<(unsigned)((n + 3) / 4), kObsThreads, 0, stream>>>(args...);
+      break;
+    case 8:
+      observe_kernel<kIndexed, kSample, kBf16, 8>
+          <<<(unsigned)((n + 7) / 8), kObsThreads, 0, stream>>>(args...);
+      break;
     case 16:
       observe_kernel<kIndexed, kSample, kBf16, 16>
           <<<(unsigned)((n + 15) / 16), kObsThreads, 0, stream>>>(args...);
@@ -1324,7 +1527,11 @@ inline void launch_observe(int64_t n, hipStream_t stream, Args... args) {
 template <int kMode, bool kEvents, class... Args>
 inline void launch_step(int64_t n, hipStream_t stream, Args... args) {
   const int rows = step_rows(n);
-  if (rows == 16) {
+  if (rows == 4) {
+    step_kernel<kMode, kEvents, 64, 4><<<(unsigned)((n + 3) / 4), 64, 0, stream>>>(args...);
+  } else if (rows == 8) {
+    step_kernel<kMode, kEvents, 64, 8><<<(unsigned)((n + 7) / 8), 64, 0, stream>>>(args...);
+  } else if (rows == 16) {
     step_kernel<kMode, kEvents, 64, 16><<<(unsigned)((n + 15) / 16), 64, 0, stream>>>(args...);
   } else if (rows == 32) {
     step_kernel<kMode, kEvents, 128, 32><<<(unsigned)((n + 31) / 32), 128, 0, stream>>>(args...);
@@ -1438,10 +1645,19 @@ int play_random(uint8_t* states, int64_t n, uint64_t* sampler, float* features,
   if (n == 0) return 0;
   const AutoReset ar{base_seed, (u64)seed_stride, generation, reinterpret_cast<u64*>(sampler),
                      reinterpret_cast<u64*>(spares), spare_gen, n, (u32)(spare_slots - 1)};
-  play_kernel<<<tiles(n), kPlayThreads, 0, stream>>>(
-      reinterpret_cast<u64*>(states), n, reinterpret_cast<u64*>(sampler), features, legal,
-      player, obs_done, obs_status, actions, reward, done, nagari, status, committed, ar,
-      (int)steps, step_rows);
+  const auto go = [&](auto kernel, int rows) {
+    kernel<<<(unsigned)((n + rows - 1) / rows), kPlayThreads, 0, stream>>>(
+        reinterpret_cast<u64*>(states), n, reinterpret_cast<u64*>(sampler), features, legal,
+        player, obs_done, obs_status, actions, reward, done, nagari, status, committed, ar,
+        (int)steps, step_rows);
+  };
+  switch (play_rows(n)) {
+    case 4: go(play_split_kernel<4>, 4); break;
+    case 8: go(play_split_kernel<8>, 8); break;
+    case 16: go(play_split_kernel<16>, 16); break;
+    case 32: go(play_split_kernel<32>, 32); break;
+    default: go(play_kernel, kTile);
+  }
   return launched();
 }
 }  // namespace
@@ -1487,10 +1703,18 @@ int cugo_branch_observe_indexed(const uint8_t* states, int64_t env_count, const 
                  !committed || !features || !legal || !player || !obs_done || !obs_status)))
     return kBadArgument;
   if (n == 0) return 0;
-  branch_observe_kernel<<<tiles(n), kPlayThreads, 0, stream>>>(
-      reinterpret_cast<const u64*>(states), env_count, ids, actions, n,
-      reinterpret_cast<u64*>(children), reward, done, nagari, status, committed, features,
-      legal, player, obs_done, obs_status);
+  const auto go = [&](auto kernel, int rows) {
+    kernel<<<(unsigned)((n + rows - 1) / rows), kPlayThreads, 0, stream>>>(
+        reinterpret_cast<const u64*>(states), env_count, ids, actions, n,
+        reinterpret_cast<u64*>(children), reward, done, nagari, status, committed, features,
+        legal, player, obs_done, obs_status);
+  };
+  switch (branch_observe_rows(n)) {
+    case 4: go(branch_observe_kernel<4>, 4); break;
+    case 16: go(branch_observe_kernel<16>, 16); break;
+    case 32: go(branch_observe_kernel<32>, 32); break;
+    default: go(branch_observe_kernel<kTile>, kTile);
+  }
   return launched();
 }
 
@@ -1529,22 +1753,25 @@ int cugo_step_observe_spares(uint8_t* states, const int64_t* actions, int64_t n,
   if (n == 0) return 0;
   const AutoReset ar{base_seed, (u64)seed_stride, generation, reinterpret_cast<u64*>(sampler),
                      reinterpret_cast<u64*>(spares), spare_gen, n, (u32)(spare_slots - 1)};
-  // Games a tile: measured on MI355X at 32,768 rows (the PPO rollout's batch), us a launch
-  // for (games, threads): (64, 128) 54.0, (32, 128) 44.2, (32, 64) 50.3, (24, 64) 50.1,
-  // (16, 64) 45.5, (16, 128) 71.9.  A wavefront runs the union of its games' rule paths, so
-  // fewer games a wavefront execute fewer divergent branches, while more wavefronts than
-  // the ~210 VGPRs let a SIMD hold (two) cost a second round.
-  constexpr int kRows = kStepObserveRows, kThreads = kPlayThreads;
-  if (features_dtype == CUGO_DTYPE_BF16)
-    step_observe_kernel<true, kRows, kThreads><<<(unsigned)((n + kRows - 1) / kRows), kThreads,
-                                                0, stream>>>(
+  // One wave a tile of 4 games, two (the second joins the staging and the stores) above:
+  // at 16,384 rows 16 games on (128 / 64) threads took 42.5 / 49.0 us with the sampler.
+  const auto go = [&](auto f32, auto bf16, int rows, int threads) {
+    (features_dtype == CUGO_DTYPE_BF16 ? bf16 : f32)<<<(unsigned)((n + rows - 1) / rows), threads,
+                                                       0, stream>>>(
         reinterpret_cast<u64*>(states), n, actions, reward, done, nagari, status, committed, ar,
         features, legal, player, obs_done, obs_status);
-  else
-    step_observe_kernel<false, kRows, kThreads><<<(unsigned)((n + kRows - 1) / kRows), kThreads,
-                                                 0, stream>>>(
-        reinterpret_cast<u64*>(states), n, actions, reward, done, nagari, status, committed, ar,
-        features, legal, player, obs_done, obs_status);
+  };
+  switch (step_observe_rows(n)) {
+    case 4: go(step_observe_kernel<false, 4, 64>, step_observe_kernel<true, 4, 64>, 4, 64); break;
+    case 16:
+      go(step_observe_kernel<false, 16, 128>, step_observe_kernel<true, 16, 128>, 16, 128);
+      break;
+    case 32:
+      go(step_observe_kernel<false, 32, 128>, step_observe_kernel<true, 32, 128>, 32, 128);
+      break;
+    default:
+      go(step_observe_kernel<false, 64, 128>, step_observe_kernel<true, 64, 128>, 64, 128);
+  }
   return launched();
 }
 
@@ -1618,10 +1845,16 @@ int cugo_branch_indexed(const uint8_t* states, int64_t env_count, const int64_t*
                  !committed)))
     return kBadArgument;
   if (n == 0) return 0;
-  branch_kernel<kTile><<<tiles(n), kTile, 0, stream>>>(reinterpret_cast<const u64*>(states),
-                                                env_count, ids, actions, n,
-                                                reinterpret_cast<u64*>(children), reward,
-                                                done, nagari, status, committed);
+  const auto go = [&](auto kernel, int rows) {
+    kernel<<<(unsigned)((n + rows - 1) / rows), kTile, 0, stream>>>(
+        reinterpret_cast<const u64*>(states), env_count, ids, actions, n,
+        reinterpret_cast<u64*>(children), reward, done, nagari, status, committed);
+  };
+  switch (branch_rows(n)) {
+    case 16: go(branch_kernel<16>, 16); break;
+    case 32: go(branch_kernel<32>, 32); break;
+    default: go(branch_kernel<kTile>, kTile);
+  }
   return launched();
 }
 
@@ -1789,8 +2022,19 @@ int cugo_rollout_canonical(const int64_t* seeds, const int64_t* first_players, i
       (n > 0 && (!seeds || !first_players || !digest)))
     return kBadArgument;
   if (n == 0) return 0;
-  canonical_kernel<<<tiles(n), kTile, 0, stream>>>(seeds, first_players, n, (u32)max_actions,
-                                                   digest);
+  const auto go = [&](auto kernel, int rows) {
+    kernel<<<(unsigned)((n + rows - 1) / rows), kTile, 0, stream>>>(seeds, first_players, n,
+                                                                    (u32)max_actions, digest);
+  };
+  switch (canonical_rows(n)) {
+    case 1: go(canonical_kernel<1>, 1); break;
+    case 2: go(canonical_kernel<2>, 2); break;
+    case 4: go(canonical_kernel<4>, 4); break;
+    case 8: go(canonical_kernel<8>, 8); break;
+    case 16: go(canonical_kernel<16>, 16); break;
+    case 32: go(canonical_kernel<32>, 32); break;
+    default: go(canonical_kernel<kTile>, kTile);
+  }
   return launched();
 }
 
