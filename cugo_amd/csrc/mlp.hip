@@ -39,6 +39,7 @@
 // Why not four wavefronts of 128 columns each: h alone would then fill the 256
 // accumulator registers a lane can address, and the compiler gives every MFMA of a kernel
 // the same accumulator file, so fc1's accumulators would have nowhere to go.
+// Batches of at most 16,384 rows run on smaller tiles (actor_rows_kernel below).
 // Arithmetic: bf16 operands, fp32 accumulation; h is kept in fp32 between blocks (the
 // layer-by-layer path rounds it to bf16), LN statistics in fp32.
 #include <hip/hip_runtime.h>
@@ -100,19 +101,21 @@ struct Weights {
   float eps;
 };
 
-// Element offset of (row r, column k) in an LDS activation tile of kM rows: K step by K
+// Element offset of (row r, column k) in an LDS activation tile of BM rows: K step by K
 // step ([k / 32][r][32]), so one MFMA A fragment (16 rows, one K step) is 1 KiB and the
 // next row tile 1 KiB further; within a row's 64 bytes, 16-byte group g sits at
 // g ^ ((r >> 1) & 3), so the 16 rows of a fragment read at one group cover every bank.
+template <int BM>
 __device__ inline int swz(int r, int k) {
-  return ((k >> 5) * kM + r) * 32 + (((((k >> 3) & 3) ^ ((r >> 1) & 3))) << 3) + (k & 7);
+  return ((k >> 5) * BM + r) * 32 + (((((k >> 3) & 3) ^ ((r >> 1) & 3))) << 3) + (k & 7);
 }
 
 // Where the accumulator layout lands in a swz() tile: element (r0 + 16 mt + 4 q4 + i,
 // c0 + 16 t + l16), r0 a multiple of 8 and c0 of 32, is at
-//   base[2 (t & 1) + (i >> 1)] + (c0 / 32 + t / 2) * 32 kM + 32 r0 + 512 mt + 32 i,
+//   base[2 (t & 1) + (i >> 1)] + (c0 / 32 + t / 2) * 32 BM + 32 r0 + 512 mt + 32 i,
 // base[c] = 128 q4 + (l16 & 7) + 8 (((2 (q4 & 1)) | (l16 >> 3)) ^ c): four lane bases and
 // static offsets, so a layer's stores hold four address registers.
+template <int BM>
 struct StoreBases {
   int base[4];
   __device__ StoreBases(int q4, int l16) {
@@ -121,7 +124,7 @@ struct StoreBases {
     for (int c = 0; c < 4; ++c) base[c] = 128 * q4 + (l16 & 7) + ((xl ^ c) << 3);
   }
   __device__ int at(int r0, int c0, int mt, int t, int i) const {
-    return base[(2 * (t & 1)) | (i >> 1)] + (c0 / 32 + t / 2) * 32 * kM + 32 * r0 + 512 * mt +
+    return base[(2 * (t & 1)) | (i >> 1)] + (c0 / 32 + t / 2) * 32 * BM + 32 * r0 + 512 * mt +
            32 * i;
   }
 };
@@ -258,19 +261,21 @@ __device__ inline void row16_sums(float (&v)[N]) {
 
 // Z[r][n] = bf16(LN(h)[r][n] * gamma[n] + beta[n]) for the wavefront's columns; every
 // wavefront calls it.  Per-row partial sums (sum, sum of squares over a wavefront's
-// columns) go to `red` (over U); after a barrier, thread r < kM turns row r's into
+// columns) go to `red` (over U); after a barrier, thread r < BM turns row r's into
 // (rstd, -mean * rstd) once; after a second barrier every lane reads its rows' pair and
 // normalises with two FMAs a value.
-__device__ inline void layer_norm(const f32x4 (&h)[kMT][kNT], const __bf16* gamma,
+template <int MT>
+__device__ inline void layer_norm(const f32x4 (&h)[MT][kNT], const __bf16* gamma,
                                   const __bf16* beta, float eps, __bf16* Z, float* red,
                                   int wave, int l16, int q4, int tid) {
-  float* stats = red + kWaves * kM * 2;  // [kM][2]
+  constexpr int BM = 16 * MT;
+  float* stats = red + kWaves * BM * 2;  // [kM][2]
   // per (row tile, row) partial sums, half the row tiles at a time; their DPP reductions
   // run stage by stage, so consecutive DPP reads never depend on the instruction just
   // before them
-  constexpr int kHalf = kMT / 2;
+  constexpr int kHalf = MT > 1 ? MT / 2 : 1;
 #pragma unroll
-  for (int half = 0; half < 2; ++half) {
+  for (int half = 0; half < MT / kHalf; ++half) {
     float a[kHalf * 4], b[kHalf * 4];
 #pragma unroll
     for (int m = 0; m < kHalf; ++m)
@@ -295,17 +300,17 @@ __device__ inline void layer_norm(const f32x4 (&h)[kMT][kNT], const __bf16* gamm
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int r = 16 * (half * kHalf + m) + 4 * q4 + i;
-          *reinterpret_cast<float2*>(red + (wave * kM + r) * 2) =
+          *reinterpret_cast<float2*>(red + (wave * BM + r) * 2) =
               make_float2(a[m * 4 + i], b[m * 4 + i]);
         }
     }
   }
   __syncthreads();
-  if (tid < kM) {
+  if (tid < BM) {
     float a = 0.f, b = 0.f;
 #pragma unroll
     for (int w = 0; w < kWaves; ++w) {
-      const float2 p = *reinterpret_cast<const float2*>(red + (w * kM + tid) * 2);
+      const float2 p = *reinterpret_cast<const float2*>(red + (w * BM + tid) * 2);
       a += p.x;
       b += p.y;
     }
@@ -316,7 +321,7 @@ __device__ inline void layer_norm(const f32x4 (&h)[kMT][kNT], const __bf16* gamm
   }
   __syncthreads();
   const int n0 = wave * (16 * kNT);
-  const StoreBases sb(q4, l16);
+  const StoreBases<BM> sb(q4, l16);
   float g[kNT], be[kNT];
 #pragma unroll
   for (int t = 0; t < kNT; ++t) {
@@ -324,7 +329,7 @@ __device__ inline void layer_norm(const f32x4 (&h)[kMT][kNT], const __bf16* gamm
     be[t] = (float)beta[n0 + 16 * t + l16];
   }
 #pragma unroll
-  for (int mt = 0; mt < kMT; ++mt)
+  for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const float2 st = *reinterpret_cast<const float2*>(stats + (16 * mt + 4 * q4 + i) * 2);
@@ -341,8 +346,9 @@ template <>
 struct Input<float> {
   // eight elements as bf16 (round to nearest even, as torch's conversion)
   __device__ static uint4 load8(const float* p) {
-    const float4 v0 = *reinterpret_cast<const float4*>(p);
-    const float4 v1 = *reinterpret_cast<const float4*>(p + 4);
+    return round8(*reinterpret_cast<const float4*>(p), *reinterpret_cast<const float4*>(p + 4));
+  }
+  __device__ static uint4 round8(float4 v0, float4 v1) {
     auto two = [](float lo, float hi) {
       return (uint32_t)__builtin_bit_cast(uint16_t, (__bf16)lo) |
              ((uint32_t)__builtin_bit_cast(uint16_t, (__bf16)hi) << 16);
@@ -381,7 +387,7 @@ __device__ inline void load_input(const TIn* __restrict__ x, __bf16* __restrict_
       const int col = c0 + 8 * (j - r * GROUPS);
       const bool valid = row0 + r < n && col < F;
       const uint4 val = valid ? v[u] : make_uint4(0u, 0u, 0u, 0u);
-      *reinterpret_cast<uint4*>(Z + swz(r, col - c0)) = val;
+      *reinterpret_cast<uint4*>(Z + swz<kM>(r, col - c0)) = val;
       if (x_copy != nullptr && valid)
         *reinterpret_cast<uint4*>(x_copy + (row0 + r) * F + col) = val;
     }
@@ -410,7 +416,7 @@ __global__ __launch_bounds__(kThreads) void actor_kernel(const TIn* __restrict__
   const int tile0 = n0 / 16;
   // fc1's grid: rows [64 wr, 64 wr + 64), chunk columns [32 wc, 32 wc + 32)
   const int wr = wave / kGridCols, wc = wave % kGridCols;
-  const StoreBases sb(q4, l16);
+  const StoreBases<kM> sb(q4, l16);
 
   auto rsrc = [](const __bf16* p, int rows, int cols) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<__bf16*>(p), (short)0, rows * cols * 2,
@@ -437,14 +443,36 @@ __global__ __launch_bounds__(kThreads) void actor_kernel(const TIn* __restrict__
     const auto w2 = rsrc(w.w2[b], kD, kD);
     // z = LN(h) -> Z.  The barriers inside come after every wavefront's last read of the
     // previous layer's input (Z) and of U, so both can be overwritten after them.
+    // The first weights of every GEMM, and fc1's bias, load before the LayerNorm, U's stores
+    // or the barrier ahead of it instead of after: 32,768 rows 125.0 -> 123.3 us.  Issued
+    // before fc2's GEMM, fc1's would spill 8 registers, for no gain.
+    bf16x8 ring1[kDepthNarrow + 1][kU_NT];
+    float bias1[kU_NT];
+    auto fill1 = [&](int c) {
+      ring_fill<kU_NT, kSteps, kDepthNarrow>(
+          ring1, BSrc(w1, kSteps, (kChunk * c + ucol) / 16, 0), lane);
+    };
+    auto fill_bias1 = [&](int c) {
+#pragma unroll
+      for (int t = 0; t < kU_NT; ++t) bias1[t] = (float)w.b1[b][kChunk * c + ucol + 16 * t + l16];
+    };
+    fill1(0);
     layer_norm(h, w.ln_w[b], w.ln_b[b], w.eps, Z, red, wave, l16, q4, tid);
+    fill_bias1(0);
     __syncthreads();  // Z complete
 #pragma unroll
     for (int c = 0; c < kChunks; ++c) {
       f32x4 u[kU_MT][kU_NT];
-      set_bias<kU_MT, kU_NT>(u, w.b1[b], kChunk * c + ucol, l16);
-      gemm<kU_MT, kU_NT, kSteps, kDepthNarrow, 2>(u, BSrc(w1, kSteps, (kChunk * c + ucol) / 16, 0),
-                                                   Z, urow, lane, l16, q4);
+#pragma unroll
+      for (int t = 0; t < kU_NT; ++t)
+#pragma unroll
+        for (int mt = 0; mt < kU_MT; ++mt)
+          u[mt][t] = f32x4{bias1[t], bias1[t], bias1[t], bias1[t]};
+      gemm_run<kU_MT, kU_NT, kSteps, kDepthNarrow, 2>(
+          u, ring1, BSrc(w1, kSteps, (kChunk * c + ucol) / 16, 0), Z, urow, lane, l16, q4);
+      const BSrc s2(w2, kSteps, tile0, c * (kChunk / kK));
+      bf16x8 ring2[kDepthWide + 1][kNT];
+      ring_fill<kNT, kChunk / kK, kDepthWide>(ring2, s2, lane);
 #pragma unroll
       for (int mt = 0; mt < kU_MT; ++mt)
 #pragma unroll
@@ -453,8 +481,9 @@ __global__ __launch_bounds__(kThreads) void actor_kernel(const TIn* __restrict__
           for (int i = 0; i < 4; ++i)
             U[sb.at(urow, ucol, mt, t, i)] = (__bf16)fmaxf(u[mt][t][i], 0.f);
       __syncthreads();  // U complete
-      gemm<kMT, kNT, kChunk / kK, kDepthWide, 1>(h, BSrc(w2, kSteps, tile0, c * (kChunk / kK)), U,
-                                                 0, lane, l16, q4);
+      gemm_run<kMT, kNT, kChunk / kK, kDepthWide, 1>(h, ring2, s2, U, 0, lane, l16, q4);
+      if (c + 1 < kChunks) fill1(c + 1);
+      if (c + 1 < kChunks) fill_bias1(c + 1);
       __syncthreads();  // U read
     }
     const __bf16* b2 = w.b2[b];
@@ -498,6 +527,244 @@ __global__ __launch_bounds__(kThreads) void actor_kernel(const TIn* __restrict__
     }
 }
 
+// ---------------------------------------------------------------- small batches ----
+// The same network on tiles of 16 MT rows (MT = 1, 2, 4) for batches that leave most CUs
+// without a 128-row tile.  A CU then runs one tile and what bounds it is its stream of all
+// 4.2 MB of weights, so the kernel keeps that stream going:
+//   * one ring of registers carries the weights of the whole network in the order they are
+//     used (3 K steps of 4 fragments a wavefront in flight, 96 KiB a CU; 7 steps measured
+//     the same): the next layer's first
+//     steps load during this layer's last ones and stay in flight through the barriers,
+//     the LayerNorm and the stores between them;
+//   * every bias and LayerNorm vector is copied into LDS at the start: a global load in
+//     between would wait for the older weight loads of the ring;
+//   * fc1 runs whole (512 columns, 64 a wavefront, as h's) instead of in four chunks: two
+//     barriers a block instead of eight, beside the LayerNorm's three.
+// Every sum is in the 128-row kernel's order, so the outputs are the same bits.  300 rows:
+// 114 -> 42 us, 42 bytes of weights a cycle on each of 19 CUs (the L1 fills 64).
+constexpr int kRing = 4;
+constexpr int kParams = kD * (1 + 2 * (kMaxBlocks + 1) + 2 * kMaxBlocks);  // + the head's
+
+template <class TIn>
+struct Raw;
+template <>
+struct Raw<float> {
+  float4 a, b;
+  __device__ void load(const float* p) {
+    a = *reinterpret_cast<const float4*>(p);
+    b = *reinterpret_cast<const float4*>(p + 4);
+  }
+  __device__ uint4 bf16() const { return Input<float>::round8(a, b); }
+};
+template <>
+struct Raw<__bf16> {
+  uint4 a;
+  __device__ void load(const __bf16* p) { a = *reinterpret_cast<const uint4*>(p); }
+  __device__ uint4 bf16() const { return a; }
+};
+
+// A layer's weights as the ring reads them: tile t's fragment of K step s at
+// o[t] + s KiB.
+struct Stream {
+  __amdgpu_buffer_rsrc_t rsrc;
+  int o[kNT];
+  __device__ Stream(const __bf16* p, int rows, int steps, int tile0, int tiles) {
+    rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<__bf16*>(p), (short)0,
+                                             rows * steps * kK * 2, 0x00020000);
+#pragma unroll
+    for (int t = 0; t < kNT; ++t) o[t] = (tile0 + t % tiles) * steps * kFrag * 2;
+  }
+  __device__ bf16x8 at(int t, int s, int lane_off) const {
+    return __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(
+                                          rsrc, lane_off, o[t] + s * kFrag * 2, 0));
+  }
+};
+
+// acc[mt][t] += A x B over NSTEPS K steps, B through the ring: step s's fragments are in
+// slot s % kRing (NSTEPS and the layers before are whole rounds of it), and while it runs the
+// step kRing - 1 ahead loads, from `next` past this layer's end.
+template <int MT, int NT, int NSTEPS>
+__device__ inline void gemm_stream(f32x4 (&acc)[MT][NT], bf16x8 (&ring)[kRing][kNT],
+                                   const Stream& cur, const Stream& next, const __bf16* A,
+                                   int lane, int l16, int q4) {
+  static_assert(NSTEPS % kRing == 0, "whole rounds of the ring");
+  constexpr int BM = 16 * MT;
+  const int a_lane = l16 * 32 + ((q4 ^ ((l16 >> 1) & 3)) << 3);
+  // the next stage's A fragments are read while this one's MFMAs issue; a stage is a whole
+  // step, or half of one at MT = 4, whose whole steps would spill
+  constexpr int AH = MT > 2 ? MT / 2 : MT;
+  constexpr int kStages = MT / AH;
+  bf16x8 a[2][AH];
+#pragma unroll
+  for (int m = 0; m < AH; ++m) a[0][m] = *reinterpret_cast<const bf16x8*>(A + a_lane + m * 512);
+#pragma unroll
+  for (int s = 0; s < NSTEPS; ++s) {
+    const int f = s + kRing - 1;
+#pragma unroll
+    for (int t = 0; t < kNT; ++t)
+      ring[f % kRing][t] = f < NSTEPS ? cur.at(t, f, lane * 16) : next.at(t, f - NSTEPS, lane * 16);
+#pragma unroll
+    for (int g = 0; g < kStages; ++g) {
+      const int stage = s * kStages + g;
+      const int next_s = (stage + 1) / kStages, next_g = (stage + 1) % kStages;
+      if (next_s < NSTEPS) {
+#pragma unroll
+        for (int m = 0; m < AH; ++m)
+          a[(stage + 1) & 1][m] = *reinterpret_cast<const bf16x8*>(
+              A + a_lane + next_s * 32 * BM + (next_g * AH + m) * 512);
+      }
+#pragma unroll
+      for (int m = 0; m < AH; ++m)
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+          acc[g * AH + m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              a[stage & 1][m], ring[s % kRing][t], acc[g * AH + m][t], 0, 0, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);  // keep the ring, as gemm_run does
+  }
+}
+
+template <class TIn, int MT>
+__global__ __launch_bounds__(kThreads) void actor_rows_kernel(
+    const TIn* __restrict__ x, __bf16* __restrict__ x_copy, int64_t n, Weights w,
+    __bf16* __restrict__ logits, float* __restrict__ value) {
+  constexpr int BM = 16 * MT;
+  // Z and U, 512 columns each; the input's 768 columns lie across both
+  __shared__ __attribute__((aligned(16))) __bf16 smem[2 * BM * kD];
+  __shared__ float red[(kWaves + 1) * BM * 2];
+  __shared__ __bf16 params[kParams + kHeadN];
+  __bf16* Z = smem;
+  __bf16* U = smem + BM * kD;
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15;
+  const int q4 = lane >> 4;
+  const int64_t row0 = (int64_t)blockIdx.x * BM;
+  const int F = w.features;
+  const int A = w.actions;
+  const int n0 = wave * (16 * kNT);
+  const int tile0 = n0 / 16;
+  const StoreBases<BM> sb(q4, l16);
+
+  // ---- x, the vectors, then the ring: all in flight together
+  constexpr int kGroups = kMaxIn / 8;
+  constexpr int kPer = BM * kGroups / kThreads;
+  static_assert(kPer * kThreads == BM * kGroups, "whole rounds");
+  Raw<TIn> xv[kPer];
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    const int j = u * kThreads + tid;
+    const int r = j / kGroups;
+    const int col = 8 * (j - r * kGroups);
+    const int64_t g = row0 + r < n ? row0 + r : n - 1;
+    xv[u].load(x + g * F + (col < F ? col : F - 8));
+  }
+  // thread t holds element t of each vector (kD threads); blocks past the network's read
+  // b_in, which is there
+  static_assert(kThreads == kD, "a thread an element");
+  constexpr int kVectors = kParams / kD;
+  __bf16 pv[kVectors + 1];
+  pv[0] = w.b_in[tid];
+#pragma unroll
+  for (int b = 0; b <= kMaxBlocks; ++b) {
+    pv[1 + 2 * b] = (b <= w.blocks ? w.ln_w[b] : w.b_in)[tid];
+    pv[2 + 2 * b] = (b <= w.blocks ? w.ln_b[b] : w.b_in)[tid];
+  }
+#pragma unroll
+  for (int b = 0; b < kMaxBlocks; ++b) {
+    pv[3 + 2 * kMaxBlocks + 2 * b] = (b < w.blocks ? w.b1[b] : w.b_in)[tid];
+    pv[4 + 2 * kMaxBlocks + 2 * b] = (b < w.blocks ? w.b2[b] : w.b_in)[tid];
+  }
+  pv[kVectors] = w.b_head[tid <= A ? tid : 0];
+  bf16x8 ring[kRing][kNT];
+  Stream cur(w.w_in, kD, kInSteps, tile0, kNT);
+#pragma unroll
+  for (int s = 0; s < kRing - 1; ++s)
+#pragma unroll
+    for (int t = 0; t < kNT; ++t) ring[s][t] = cur.at(t, s, lane * 16);
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    const int j = u * kThreads + tid;
+    const int r = j / kGroups;
+    const int col = 8 * (j - r * kGroups);
+    const bool valid = row0 + r < n && col < F;
+    const uint4 val = valid ? xv[u].bf16() : make_uint4(0u, 0u, 0u, 0u);
+    *reinterpret_cast<uint4*>(smem + swz<BM>(r, col)) = val;
+    if (x_copy != nullptr && valid)
+      *reinterpret_cast<uint4*>(x_copy + (row0 + r) * F + col) = val;
+  }
+#pragma unroll
+  for (int v = 0; v < kVectors; ++v) params[v * kD + tid] = pv[v];
+  if (tid < kHeadN) params[kParams + tid] = tid <= A ? pv[kVectors] : (__bf16)0.f;
+  __syncthreads();
+
+  const __bf16* ln = params + kD;  // [block][weight, bias]
+  const __bf16* bias = ln + 2 * (kMaxBlocks + 1) * kD;  // [block][b1, b2]
+  const Stream head(w.w_head, kHeadN, kSteps, wave * kHeadNT, kHeadNT);
+  // the layer after the input or a block: the next block's fc1 or the head
+  auto after = [&](int b) {
+    return b < w.blocks ? Stream(w.w1[b], kD, kSteps, tile0, kNT) : head;
+  };
+  f32x4 h[MT][kNT];
+  set_bias<MT, kNT>(h, params, n0, l16);
+  Stream next = after(0);
+  gemm_stream<MT, kNT, kInSteps>(h, ring, cur, next, smem, lane, l16, q4);
+  __syncthreads();  // the input is read: Z is written next
+  for (int b = 0; b < w.blocks; ++b) {
+    cur = next;
+    // Between two writes of one buffer lie barriers past its reads: Z is read by fc1,
+    // before the barrier that completes U, and U by fc2, before the LayerNorm's.
+    layer_norm<MT>(h, ln + 2 * b * kD, ln + (2 * b + 1) * kD, w.eps, Z, red, wave, l16, q4, tid);
+    __syncthreads();  // Z complete
+    f32x4 u[MT][kNT];
+    set_bias<MT, kNT>(u, bias + 2 * b * kD, n0, l16);
+    const Stream w2(w.w2[b], kD, kSteps, tile0, kNT);
+    gemm_stream<MT, kNT, kSteps>(u, ring, cur, w2, Z, lane, l16, q4);
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int t = 0; t < kNT; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) U[sb.at(0, n0, mt, t, i)] = (__bf16)fmaxf(u[mt][t][i], 0.f);
+    __syncthreads();  // U complete
+    next = after(b + 1);
+    gemm_stream<MT, kNT, kSteps>(h, ring, w2, next, U, lane, l16, q4);
+    const __bf16* b2 = bias + (2 * b + 1) * kD;
+#pragma unroll
+    for (int t = 0; t < kNT; ++t) {
+      const float v = (float)b2[n0 + 16 * t + l16];
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) h[mt][t] += f32x4{v, v, v, v};
+    }
+  }
+
+  // ---- head, as the 128-row kernel's
+  const int hn0 = wave * (16 * kHeadNT);
+  layer_norm<MT>(h, ln + 2 * w.blocks * kD, ln + (2 * w.blocks + 1) * kD, w.eps, Z, red, wave, l16,
+                 q4, tid);
+  __syncthreads();  // Z complete
+  f32x4 o[MT][kHeadNT];
+  set_bias<MT, kHeadNT>(o, params + kParams, hn0, l16);
+  gemm_stream<MT, kHeadNT, kSteps>(o, ring, head, head, Z, lane, l16, q4);
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int64_t r = row0 + 16 * mt + 4 * q4 + i;
+      if (r >= n) continue;
+#pragma unroll
+      for (int t = 0; t < kHeadNT; ++t) {
+        const int col = hn0 + 16 * t + l16;
+        if (col < A)
+          logits[r * A + col] = (__bf16)o[mt][t][i];
+        else if (col == A)
+          value[r] = o[mt][t][i];
+      }
+    }
+}
+
 // packed[((tile * steps + step) * 64 + (q * 16 + r)) * 8 + i] = w[16 tile + r][32 step +
 // 8 q + i], zero outside [rows, cols): one thread per packed element.
 __global__ void pack_kernel(const __bf16* __restrict__ w, int64_t rows, int64_t cols,
@@ -514,6 +781,32 @@ __global__ void pack_kernel(const __bf16* __restrict__ w, int64_t rows, int64_t 
   const int64_t rr = tile * 16 + (l & 15);
   const int64_t cc = step * kK + 8 * (l >> 4) + i;
   packed[j] = (rr < rows && cc < cols) ? w[rr * cols + cc] : (__bf16)0.f;
+}
+
+template <class TIn>
+int launch_actor(const TIn* x, __bf16* x_copy, int64_t n, const Weights& w, __bf16* logits,
+                 float* value, hipStream_t stream) {
+  auto grid = [&](int rows) { return dim3((unsigned)((n + rows - 1) / rows)); };
+  // A tile's time hardly depends on how many CUs hold one until the whole chip streams the
+  // weights: the smallest tile that leaves a CU at most one.  us at 128 / 64 / 32 / 16 rows
+  // (float32 rows): 300 rows 114 / 57 / 47 / 42; 3,000: 115 / 57 / 46 / 46; 4,096: 114 / 57 /
+  // 47 / 51 (256 tiles of 16 rows: the weights' stream from L2 slows down past ~192);
+  // 8,192: 115 / 58 / 56 / 100; 16,384: 123 / 73 / 110 / 198; 32,768, where 64-row tiles take
+  // two rounds, 137 / 140.
+  constexpr int kCUs = 256;
+#define CUGO_ACTOR(KERNEL, ROWS) \
+  hipLaunchKernelGGL((KERNEL), grid(ROWS), dim3(kThreads), 0, stream, x, x_copy, n, w, logits, value)
+  if (n <= 16 * (kCUs * 3 / 4)) {
+    CUGO_ACTOR((actor_rows_kernel<TIn, 1>), 16);
+  } else if (n <= 32 * kCUs) {
+    CUGO_ACTOR((actor_rows_kernel<TIn, 2>), 32);
+  } else if (n <= 64 * kCUs) {
+    CUGO_ACTOR((actor_rows_kernel<TIn, 4>), 64);
+  } else {
+    CUGO_ACTOR((actor_kernel<TIn>), kM);
+  }
+#undef CUGO_ACTOR
+  return (int)hipGetLastError();
 }
 
 }  // namespace mlp
@@ -567,20 +860,14 @@ extern "C" int cugo_mlp_actor_forward(int x_dtype, const void* x, void* x_copy, 
   w.features = src.features;
   w.actions = src.actions;
   w.eps = src.eps;
-  const unsigned grid = (unsigned)((n + kM - 1) / kM);
   auto* xc = static_cast<__bf16*>(x_copy);
   auto* lg = static_cast<__bf16*>(logits);
   switch (x_dtype) {
     case CUGO_DTYPE_F32:
-      hipLaunchKernelGGL(actor_kernel<float>, dim3(grid), dim3(kThreads), 0, stream,
-                         static_cast<const float*>(x), xc, n, w, lg, value);
-      break;
+      return launch_actor(static_cast<const float*>(x), xc, n, w, lg, value, stream);
     case CUGO_DTYPE_BF16:
-      hipLaunchKernelGGL(actor_kernel<__bf16>, dim3(grid), dim3(kThreads), 0, stream,
-                         static_cast<const __bf16*>(x), xc, n, w, lg, value);
-      break;
+      return launch_actor(static_cast<const __bf16*>(x), xc, n, w, lg, value, stream);
     default:
       return -2;
   }
-  return (int)hipGetLastError();
 }
