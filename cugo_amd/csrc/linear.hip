@@ -85,8 +85,44 @@ __device__ inline uint4 add_bf16(uint4 a, uint4 b) {
   return __builtin_bit_cast(uint4, z);
 }
 
-__device__ inline float gelu(float v) {
+// torch's exact GELU, x / 2 (1 + erf(x / sqrt 2)).
+__device__ inline float gelu_erf(float v) {
   return v * 0.5f * (1.0f + erff(v * 0.70710678118654752440f));
+}
+
+// gelu_erf of four bf16 values rounded to bf16, the same bits on every bf16 input, without
+// erff's branches: x Phi(x) = max(x, 0) - |x| Q(|x|) with Q the normal upper tail as
+// exp2(p(|x|)); log2 Q is smooth, and p is its weighted minimax polynomial on [0, 5.5]
+// (before the rounding within 1.3e-7 of 64 bits on [-4, 4]; erff's form 2.1e-7).  Below -4
+// erff's form loses its digits in 1 + erf, and those are the digits that torch stores: a
+// wavefront with such an input takes it.  Inputs of 2^-100 and less are halved, which is
+// their GELU.
+// A layer's tail (out_proj and feed-forward), us with erff / with this: 500 rows 15.6 / 14.4,
+// 8,192 rows 26.8 / 25.0, 12,288 rows 35.5 / 34.1.
+__device__ inline bf16x4 gelu4(bf16x4 in) {
+  constexpr float c[9] = {-0.999999344f,    -1.15113306f,     -0.459020108f,
+                          -0.0529759042f,   0.00765961129f,   -0.000535962172f,
+                          -3.95785901e-05f, 1.16156007e-05f,  -7.2305204e-07f};
+  bf16x4 out;
+  bool tail = false;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float x = (float)in[e];
+    const float z = fminf(fabsf(x), 5.5f);
+    float p = c[8];
+#pragma unroll
+    for (int i = 7; i >= 0; --i) p = __builtin_fmaf(p, z, c[i]);
+    // past 5.5 z Q is under half a bf16 step of x; -x keeps NaN
+    const float y =
+        __builtin_fmaf(x > 0.f ? -z : x, __builtin_amdgcn_exp2f(p), fmaxf(x, 0.f));
+    out[e] = (__bf16)(fabsf(x) < 0x1p-100f ? 0.5f * x : y);
+    tail = tail || x < -4.f;
+  }
+  if (tail) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) out[e] = (__bf16)gelu_erf((float)in[e]);
+  }
+  return out;
 }
 
 // Element offset of (row r, column k) in the LDS X panel of BM rows: K step major
@@ -240,10 +276,8 @@ __global__ __launch_bounds__(64 * WR * WC) void linear_kernel(Args a) {
     for (int t = 0; t < TN; ++t) {
       bf16x4 out;
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const __bf16 v = (__bf16)(acc[i][t][c] + bias[t][c]);
-        out[c] = ACT == CUGO_LINEAR_GELU ? (__bf16)gelu((float)v) : v;
-      }
+      for (int c = 0; c < 4; ++c) out[c] = (__bf16)(acc[i][t][c] + bias[t][c]);
+      if constexpr (ACT == CUGO_LINEAR_GELU) out = gelu4(out);
       const int r = r0 + 16 * i + l16, c = wc * 16 * TN + 16 * t + 4 * q4;
       *reinterpret_cast<bf16x4*>(xs + r * kOutStride + c) = out;
     }
@@ -403,11 +437,10 @@ int launch(const Args& base, int k, int act, hipStream_t stream) {
 // outputs are the same bits.
 // What bounds it: each workgroup streams all 1 MiB of W1 and W2 (and W_o's 128 KiB)
 // through its CU's L1 (the FLOPs a weight byte buys are the tile's rows), ~20 bytes a
-// cycle a CU when every CU reads the same weights at once; the GELU's erff is ~5 us of
-// VALU at 12,288 rows (the launch without it: 20.5 against 26.1 us).  A GELU table in LDS
-// (gelu() of the 4,736 bf16 inputs without a closed form, built by each workgroup, then
-// looked up; the same bits on every finite input) made the launch slower: 39.6 against
-// 31.9 us at 12,288 rows.
+// cycle a CU when every CU reads the same weights at once, beside the GELU's VALU work (see
+// gelu4).  A GELU table in LDS (of the 4,736 bf16 inputs without a closed form, built by
+// each workgroup, then looked up; the same bits on every finite input) made the launch
+// slower with erff: 39.6 against 31.9 us at 12,288 rows.
 // Weights: linear_kernel's packed fragments, W1 [1,024, 256] (8 K steps a 16-row tile)
 // and W2 [256, 1,024] (32 K steps a tile), read through buffer loads a few K steps ahead
 // of the MFMAs.
@@ -707,10 +740,8 @@ __global__ __launch_bounds__(kThreads) void ffn_kernel(Args a) {
         const int i = s / 2, t = s % 2;
         bf16x4_t o;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const __bf16 v = (__bf16)(u[gc & 1][i][t][e] + (float)b1v[t][e]);
-          o[e] = (__bf16)gelu((float)v);
-        }
+        for (int e = 0; e < 4; ++e) o[e] = (__bf16)(u[gc & 1][i][t][e] + (float)b1v[t][e]);
+        o = gelu4(o);
         *reinterpret_cast<bf16x4_t*>(us + (gc & 1) * kPanel +
                                      xs_at<BM>(16 * i + l16, c0 + 16 * t + 4 * q4)) = o;
       }
