@@ -365,8 +365,17 @@ struct PhiloxNoise {
 // the reductions follow gumbel_kernel (the largest value, the first index among equal
 // ones); only the order of the fp32 softmax sum differs.  kNoise: 0 no noise (greedy),
 // 1 the uniforms u [n, A], 2 uniforms drawn here from Philox (PhiloxNoise).
+// With Philox the arithmetic bounds it (three blocks of ten rounds, 24 logarithms and 12
+// exponentials a lane for 192 actions), and a game row has about ten legal actions: the
+// row's legal actions are packed through LDS and a lane draws for one or two of them, one
+// block and two logarithms each.  A wavefront takes this way when each of its rows has at
+// most kGumbelPacked legal actions, all logits above -1e29 (so that no illegal action's
+// -1e30 can win or be the maximum) and no uniforms are asked for; any other takes all the
+// actions.  The exponentials go back through LDS to the lanes that hold the actions, which
+// sum them in the order of the other way: the same bits.
 constexpr int kGumbelLanes = 16;
 constexpr int kGumbelPer = 12;  // up to 192 actions
+constexpr int kGumbelPacked = 2 * kGumbelLanes;
 static_assert(kGumbelPer == 12, "a Philox lane draws three blocks of four uniforms");
 
 template <class T, int kNoise>
@@ -397,6 +406,80 @@ __global__ __launch_bounds__(256) void gumbel_rows_kernel(
   if constexpr (kNoise == 2) {
     const uint32_t epoch = (uint32_t)*px.epoch;
     const uint32_t row_hi = (uint32_t)((uint64_t)rr >> 32) << 8;
+    __shared__ uint2 packed[256 / kGumbelLanes][kGumbelPacked];  // action, logit
+    uint2* slots = packed[threadIdx.x / kGumbelLanes];
+    const int shift = threadIdx.x & (64 - kGumbelLanes);  // the row's bits of a ballot
+    int count = 0;  // the row's legal actions
+    int at[kGumbelPer];  // where this lane's are packed; -1: not legal
+    bool plain = true;
+#pragma unroll
+    for (int k = 0; k < kGumbelPer; ++k) {
+      const int a = j + kGumbelLanes * k;
+      const bool legal_a = row_ok && a < actions_count && gb[k] != 0;
+      const float x = T::to_float(lv[k]);
+      plain = plain && (!legal_a || x > -1.0e29f);
+      const uint32_t bits = (uint32_t)(__ballot(legal_a) >> shift) & ((1u << kGumbelLanes) - 1);
+      at[k] = legal_a ? count + __popc(bits & ((1u << j) - 1)) : -1;
+      if (legal_a && at[k] < kGumbelPacked)
+        slots[at[k]] = make_uint2((uint32_t)a, __float_as_uint(x));
+      count += __popc(bits);
+    }
+    if (px.u_out == nullptr && __ballot(!plain || count > kGumbelPacked) == 0) {
+      // a row is one wavefront's: its own writes, read back in order
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      float mp[2] = {0.f, 0.f};
+      bool has[2] = {false, false};
+      float best = -INFINITY, best_m = -1.0e30f, top = -1.0e30f;
+      int best_a = 1 << 30;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int mine = j + kGumbelLanes * i;
+        has[i] = mine < count;
+        if (__ballot(has[i]) == 0) break;
+        if (!has[i]) continue;
+        const uint2 s = slots[mine];
+        const uint32_t a = s.x;
+        mp[i] = __uint_as_float(s.y);
+        const Philox4 w = philox4x32_10((uint32_t)rr, (a & 15u) + 64u * (a >> 6) + row_hi,
+                                        px.offset, epoch, px.k0, px.k1);
+        const uint32_t lo = a & 16u ? w.x[1] : w.x[0], hi = a & 16u ? w.x[3] : w.x[2];
+        const float u0 = (float)((a & 32u ? hi : lo) >> 8) * 0x1.0p-24f;
+        const float v = mp[i] + -logf(-logf(fminf(fmaxf(u0, 1.0e-20f), 1.0f)));
+        if (v > best) { best = v; best_a = (int)a; best_m = mp[i]; }
+        top = fmaxf(top, mp[i]);
+      }
+      for (int off = kGumbelLanes / 2; off > 0; off >>= 1) {
+        const float ob = __shfl_xor(best, off);
+        const int oa = __shfl_xor(best_a, off);
+        const float om = __shfl_xor(best_m, off);
+        if (ob > best || (ob == best && oa < best_a)) { best = ob; best_a = oa; best_m = om; }
+        top = fmaxf(top, __shfl_xor(top, off));
+      }
+      float sum = 0.0f;
+      if (logp != nullptr) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          if (has[i]) slots[j + kGumbelLanes * i].y = __float_as_uint(expf(mp[i] - top));
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+        for (int k = 0; k < kGumbelPer; ++k) {
+          const float e = __uint_as_float(slots[at[k] < 0 ? 0 : at[k]].y);
+          sum += at[k] < 0 ? 0.0f : e;
+        }
+        for (int off = kGumbelLanes / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
+      }
+      if (j == 0 && row_ok) {
+        // no legal action: the first of equal -1e30s, its share of A equal terms
+        actions[r] = count > 0 ? best_a : 0;
+        if (logp != nullptr)
+          logp[r] = count > 0 ? (best_m - top) - logf(sum) : -logf((float)actions_count);
+      }
+      return;
+    }
 #pragma unroll
     for (int g = 0; g < kGumbelPer / 4; ++g) {
       const Philox4 w = philox4x32_10((uint32_t)rr, (uint32_t)(j + 64 * g) + row_hi, px.offset,

@@ -1,0 +1,50 @@
+"""The Gumbel-max draw over a row's legal actions alone against the draw over all of them."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda"
+
+
+@pytest.fixture(scope="module")
+def ext():
+    from cugo_amd import load_extension
+
+    return load_extension()
+
+
+def _legal(n, a, counts, g):
+    """counts[r % len(counts)] legal actions in row r (at most a)."""
+    rank = torch.rand(n, a, generator=g, device=DEV).argsort(1).argsort(1)
+    want = torch.tensor([counts[r % len(counts)] for r in range(n)], device=DEV)
+    return rank < want[:, None]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,a", [(4099, 179), (1, 179), (67, 192), (130, 16), (130, 15), (9, 1)])
+def test_gumbel_packed_rows(ext, dtype, n, a):
+    """Actions and log-probabilities of gumbel_sample_philox, which packs rows of few legal
+    actions, against gumbel_sample on the same uniforms, which never does: the same bits, at
+    0 to 33 legal actions a row (33 is past the packing), mixed within wavefronts and alike
+    in them, with ties, infinities and the type's lowest value among the logits."""
+    g = torch.Generator(device=DEV).manual_seed(n + a)
+    epoch = torch.tensor([7], dtype=torch.int64, device=DEV)
+    low = torch.finfo(dtype).min
+    for counts in ([0], [1], [3, 16, 17, 31], [32], [5, 5, 5, 33], [0, 1, 2, 12]):
+        legal = _legal(n, a, counts, g)
+        for special in (None, 0.0, float("inf"), float("-inf"), low, -2e29):
+            logits = (torch.randn(n, a, generator=g, device=DEV) * 3).to(dtype)
+            if special is not None:
+                hit = torch.rand(n, a, generator=g, device=DEV) < 0.5
+                logits = torch.where(hit, torch.full_like(logits, special), logits)
+            u = torch.empty((n, a), device=DEV)
+            ext.gumbel_sample_philox(logits, legal, 99, epoch, 3, uniforms_out=u)
+            want_a, want_lp = ext.gumbel_sample(logits, legal, u)
+            got_a, got_lp = ext.gumbel_sample_philox(logits, legal, 99, epoch, 3)
+            assert torch.equal(got_a, want_a), (counts, special)
+            assert torch.equal(torch.nan_to_num(got_lp, nan=7.0),
+                               torch.nan_to_num(want_lp, nan=7.0)), (counts, special)
