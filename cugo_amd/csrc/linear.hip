@@ -93,34 +93,34 @@ __device__ inline float gelu_erf(float v) {
 // gelu_erf of four bf16 values rounded to bf16, the same bits on every bf16 input, without
 // erff's branches: x Phi(x) = max(x, 0) - |x| Q(|x|) with Q the normal upper tail as
 // exp2(p(|x|)); log2 Q is smooth, and p is its weighted minimax polynomial on [0, 5.5]
-// (before the rounding within 1.3e-7 of 64 bits on [-4, 4]; erff's form 2.1e-7).  Below -4
-// erff's form loses its digits in 1 + erf, and those are the digits that torch stores: a
-// wavefront with such an input takes it.  Inputs of 2^-100 and less are halved, which is
-// their GELU.
-// A layer's tail (out_proj and feed-forward), us with erff / with this: 500 rows 15.6 / 14.4,
-// 8,192 rows 26.8 / 25.0, 12,288 rows 35.5 / 34.1.
+// (before the rounding within 2.4e-7 of 64 bits on [-4, 4], erff's form 2.2e-7; degree 8
+// reaches 1.3e-7, and every bf16 result is the same).  Below -4 erff's form loses its digits
+// in 1 + erf, and those are the digits that torch stores: a wavefront with such an input
+// takes it, and so does one with an input under 2^-100 (0 among them), whose half has to
+// stay exact.
+// A layer's tail (out_proj and feed-forward), us with erff / with this: 500 rows 15.6 / 14.2,
+// 8,192 rows 26.8 / 23.5, 12,288 rows 35.5 / 30.8 (34.1 at degree 8 with a test an input).
 __device__ inline bf16x4 gelu4(bf16x4 in) {
-  constexpr float c[9] = {-0.999999344f,    -1.15113306f,     -0.459020108f,
-                          -0.0529759042f,   0.00765961129f,   -0.000535962172f,
-                          -3.95785901e-05f, 1.16156007e-05f,  -7.2305204e-07f};
+  constexpr float c[7] = {-0.999999523f,  -1.15115833f,    -0.458842337f, -0.0533830822f,
+                          0.00809392985f, -0.00078024494f, 3.49227848e-05f};
   bf16x4 out;
-  bool tail = false;
+  float x[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    const float x = (float)in[e];
-    const float z = fminf(fabsf(x), 5.5f);
-    float p = c[8];
+    x[e] = (float)in[e];
+    const float z = fminf(fabsf(x[e]), 5.5f);  // past 5.5 z Q is under half a bf16 step of x
+    float p = c[6];
 #pragma unroll
-    for (int i = 7; i >= 0; --i) p = __builtin_fmaf(p, z, c[i]);
-    // past 5.5 z Q is under half a bf16 step of x; -x keeps NaN
-    const float y =
-        __builtin_fmaf(x > 0.f ? -z : x, __builtin_amdgcn_exp2f(p), fmaxf(x, 0.f));
-    out[e] = (__bf16)(fabsf(x) < 0x1p-100f ? 0.5f * x : y);
-    tail = tail || x < -4.f;
+    for (int i = 5; i >= 0; --i) p = __builtin_fmaf(p, z, c[i]);
+    const float relu = __builtin_fmaf(0.5f, x[e], 0.5f * fabsf(x[e]));  // exact, keeps NaN
+    out[e] = (__bf16)__builtin_fmaf(-z, __builtin_amdgcn_exp2f(p), relu);
   }
-  if (tail) {
+  const float low = fminf(fminf(x[0], x[1]), fminf(x[2], x[3]));
+  const float small =
+      fminf(fminf(fabsf(x[0]), fabsf(x[1])), fminf(fabsf(x[2]), fabsf(x[3])));
+  if (low < -4.f || small < 0x1p-100f) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) out[e] = (__bf16)gelu_erf((float)in[e]);
+    for (int e = 0; e < 4; ++e) out[e] = (__bf16)gelu_erf(x[e]);
   }
   return out;
 }
