@@ -1198,6 +1198,31 @@ std::vector<torch::Tensor> out_proj_ffn(torch::Tensor att, torch::Tensor x,
   return ffn_impl(att, x, w1_packed, b1, w2_packed, b2, ln_weight, ln_bias, eps, rows, out, &op);
 }
 
+// cached_layer(h, x, in_packed, in_bias, heads, keys, values, pos, rows, order, then
+// out_proj_ffn's arguments from wo_packed to eps) -> as out_proj_ffn: a pre-norm layer of one
+// token a row (python/cugo_seq50.py:310-322), h = norm1(x): linear, decode_attention_append
+// on its q, k and v in place, out_proj_ffn.  One call instead of three with the views between
+// them: below ~5,000 rows the host's work, not the launches, is a layer's time (500 rows 51.4 ->
+// 35.2 us a layer, with the fewer parameter lookups of its caller).
+std::vector<torch::Tensor> cached_layer(
+    torch::Tensor h, torch::Tensor x, torch::Tensor in_packed, c10::optional<torch::Tensor> in_bias,
+    int64_t heads, torch::Tensor keys, torch::Tensor values, torch::Tensor pos,
+    c10::optional<torch::Tensor> rows, c10::optional<torch::Tensor> order,
+    torch::Tensor wo_packed, torch::Tensor bo, torch::Tensor ln2_weight, torch::Tensor ln2_bias,
+    double eps2, torch::Tensor w1_packed, torch::Tensor b1, torch::Tensor w2_packed,
+    torch::Tensor b2, c10::optional<torch::Tensor> ln_weight, c10::optional<torch::Tensor> ln_bias,
+    double eps) {
+  TORCH_CHECK(h.dim() == 2 && heads > 0 && h.size(1) % heads == 0,
+              "h must be [n, d], d a multiple of heads");
+  const int64_t n = h.size(0), d = h.size(1), dh = d / heads;
+  const auto qkv = linear(h, in_packed, 3 * d, in_bias, false, 0, c10::nullopt, c10::nullopt);
+  auto part = [&](int64_t i) { return qkv.as_strided({n, heads, dh}, {3 * d, dh, 1}, i * d); };
+  const auto att = decode_attention_append(part(0), part(1), part(2), keys, values, pos, rows,
+                                           c10::nullopt, order);
+  return out_proj_ffn(att.view({n, d}), x, wo_packed, bo, ln2_weight, ln2_bias, eps2, w1_packed,
+                      b1, w2_packed, b2, ln_weight, ln_bias, eps, 0, c10::nullopt);
+}
+
 // paired_select(active, status, done, any_legal, player, a_seat, act_a, act_b, bad,
 // any_active, playing=None) -> actions int64 [n]; paired_update(active, step_status,
 // new_done, reward0, nagari, final_reward0, final_nagari, bad, any_active, steps,
@@ -1866,6 +1891,14 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         pybind11::arg("ln_weight") = pybind11::none(), pybind11::arg("ln_bias") = pybind11::none(),
         pybind11::arg("eps") = 1e-5, pybind11::arg("rows") = 0,
         pybind11::arg("out") = pybind11::none());
+  m.def("cached_layer", &cached_layer, pybind11::arg("h"), pybind11::arg("x"), pybind11::arg("in_packed"),
+        pybind11::arg("in_bias"), pybind11::arg("heads"), pybind11::arg("keys"), pybind11::arg("values"), pybind11::arg("pos"),
+        pybind11::arg("rows"), pybind11::arg("order"), pybind11::arg("wo_packed"), pybind11::arg("bo"),
+        pybind11::arg("ln2_weight"), pybind11::arg("ln2_bias"), pybind11::arg("eps2"), pybind11::arg("w1_packed"),
+        pybind11::arg("b1"), pybind11::arg("w2_packed"), pybind11::arg("b2"), pybind11::arg("ln_weight"),
+        pybind11::arg("ln_bias"), pybind11::arg("eps"),
+        "One pre-norm layer over one token a row: in_proj, KV append + attention, out_proj and "
+        "feed-forward.");
   m.def("out_proj_ffn", &out_proj_ffn,
         "out_proj + residual add + norm2, then ffn, in one launch",
         pybind11::arg("att"), pybind11::arg("x"), pybind11::arg("wo_packed"), pybind11::arg("bo"),

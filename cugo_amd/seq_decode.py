@@ -61,8 +61,7 @@ def add_norm(x: torch.Tensor, y: torch.Tensor | None, norm: nn.Module):
             and x.dim() == 2 and x.dtype in (torch.bfloat16, torch.float32)
             and norm.weight.dtype == x.dtype and tuple(norm.normalized_shape) == (x.shape[1],)
             and x.shape[1] in _FUSED_WIDTHS and (y is None or y.dtype == x.dtype)):
-        out = _ext().add_layernorm(x.contiguous(), y, norm.weight.detach(), norm.bias.detach(),
-                                   norm.eps)
+        out = _ext().add_layernorm(x.contiguous(), y, norm.weight, norm.bias, norm.eps)
         return out[0], out[1]
     x = x if y is None else x + y
     return x, norm(x)
@@ -159,22 +158,30 @@ def linear_add_norm(u: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | 
     return add_norm(x, linear(u, weight, bias), norm)
 
 
-def _fits_ffn(layer, h: torch.Tensor, x: torch.Tensor, norm: nn.Module | None) -> bool:
-    """The shapes `ffn` takes: bf16 rows 256 wide, a 1,024-wide hidden layer with the exact
-    GELU, and (when given) an affine bf16 LayerNorm over 256 columns."""
-    l1, l2 = layer.linear1, layer.linear2
-    return (h.dim() == 2 and h.is_cuda and h.dtype == torch.bfloat16 and h.shape[1] == 256
+def _ffn_args(layer, h: torch.Tensor, x: torch.Tensor, norm: nn.Module | None) -> tuple | None:
+    """`ffn`'s arguments from w1_packed to eps, but for the weights' packing, if it takes the
+    layer: bf16 rows 256 wide, a 1,024-wide hidden layer with the exact GELU, and (when given)
+    an affine bf16 LayerNorm over 256 columns."""
+    bf16 = torch.bfloat16
+    if not (h.dim() == 2 and h.is_cuda and h.dtype == bf16 and h.shape[1] == 256
             and h.stride(1) == 1 and (h.shape[0] <= 1 or h.stride(0) % 8 == 0)
-            and h.data_ptr() % 16 == 0 and x.dtype == torch.bfloat16 and x.is_contiguous()
-            and x.shape == h.shape and is_exact_gelu(layer.activation)
-            and tuple(l1.weight.shape) == (1024, 256) and tuple(l2.weight.shape) == (256, 1024)
-            and l1.weight.dtype == torch.bfloat16 and l2.weight.dtype == torch.bfloat16
-            and l1.bias is not None and l2.bias is not None
-            and l1.bias.dtype == torch.bfloat16 and l2.bias.dtype == torch.bfloat16
-            and (norm is None or (isinstance(norm, nn.LayerNorm) and norm.weight is not None
-                                  and norm.bias is not None
-                                  and norm.weight.dtype == torch.bfloat16
-                                  and tuple(norm.normalized_shape) == (256,))))
+            and h.data_ptr() % 16 == 0 and x.dtype == bf16 and x.is_contiguous()
+            and x.shape == h.shape and is_exact_gelu(layer.activation)):
+        return None
+    l1, l2 = layer.linear1, layer.linear2  # each parameter once: a module's lookup is slow
+    w1, b1, w2, b2 = l1.weight, l1.bias, l2.weight, l2.bias
+    if not (w1.shape == (1024, 256) and w2.shape == (256, 1024) and w1.dtype == bf16
+            and w2.dtype == bf16 and b1 is not None and b2 is not None and b1.dtype == bf16
+            and b2.dtype == bf16):
+        return None
+    if norm is None:
+        return w1, b1, w2, b2, None, None, 1e-5
+    if not isinstance(norm, nn.LayerNorm):
+        return None
+    w, b = norm.weight, norm.bias
+    if w is None or b is None or w.dtype != bf16 or tuple(norm.normalized_shape) != (256,):
+        return None
+    return w1, b1, w2, b2, w, b, norm.eps
 
 
 def feed_forward(layer, h: torch.Tensor, x: torch.Tensor, norm: nn.Module | None = None):
@@ -183,13 +190,10 @@ def feed_forward(layer, h: torch.Tensor, x: torch.Tensor, norm: nn.Module | None
     returns x_out, or (x_out, norm(x_out)).  One HIP launch (`ffn`, the hidden layer kept
     on chip) for the d = 256, 1,024-wide bf16 layer; linear (GELU) and linear_add_norm /
     linear with the residual otherwise, which give the same bits."""
-    if _fits_ffn(layer, h, x, norm):
-        l1, l2 = layer.linear1, layer.linear2
-        out = _ext().ffn(h, x, packed_weight(l1.weight), l1.bias.detach(),
-                         packed_weight(l2.weight), l2.bias.detach(),
-                         None if norm is None else norm.weight.detach(),
-                         None if norm is None else norm.bias.detach(),
-                         1e-5 if norm is None else norm.eps)
+    args = _ffn_args(layer, h, x, norm)
+    if args is not None:
+        w1, b1, w2, b2, *rest = args
+        out = _ext().ffn(h, x, packed_weight(w1), b1, packed_weight(w2), b2, *rest)
         return out[0] if norm is None else (out[0], out[1])
     if is_exact_gelu(layer.activation):
         u = linear(h, layer.linear1.weight, layer.linear1.bias, gelu=True)
@@ -200,28 +204,57 @@ def feed_forward(layer, h: torch.Tensor, x: torch.Tensor, norm: nn.Module | None
     return linear_add_norm(u, layer.linear2.weight, layer.linear2.bias, x, norm)
 
 
+def _tail_args(layer, att: torch.Tensor, x: torch.Tensor, norm: nn.Module | None) -> tuple | None:
+    """`out_proj_ffn`'s arguments from wo_packed to eps, if it takes the layer: `ffn`'s with a
+    biased out_proj and an affine bf16 norm2."""
+    args = _ffn_args(layer, att, x, norm)
+    op, n2 = layer.self_attn.out_proj, layer.norm2
+    if args is None or not isinstance(n2, nn.LayerNorm):
+        return None
+    wo, bo, w, b = op.weight, op.bias, n2.weight, n2.bias
+    bf16 = torch.bfloat16
+    if not (wo.shape == (256, 256) and bo is not None and _fits_linear(att, wo, bo)
+            and w is not None and b is not None and w.dtype == bf16 and b.dtype == bf16
+            and tuple(n2.normalized_shape) == (256,)):
+        return None
+    w1, b1, w2, b2, *rest = args
+    return (packed_weight(wo), bo, w, b, n2.eps, packed_weight(w1), b1, packed_weight(w2), b2,
+            *rest)
+
+
+def _layer(layer, h: torch.Tensor, x: torch.Tensor, heads: int, keys: torch.Tensor,
+           values: torch.Tensor, pos: torch.Tensor, rows: torch.Tensor | None,
+           order: torch.Tensor | None, norm: nn.Module | None):
+    """One pre-norm layer over one token a row, h = norm1(x) (python/cugo_seq50.py:310-322):
+    attention_tail of the decode of in_proj(h), whose keys and values are appended.  One call
+    (`cached_layer`) where the three launches' operations take the layer."""
+    sa = layer.self_attn
+    w, b = sa.in_proj_weight, sa.in_proj_bias
+    n, d = x.shape
+    # h has the attention output's shape, type and layout
+    args = _tail_args(layer, h, x, norm)
+    if (args is not None and _fits_linear(h, w, b) and w.shape == (3 * d, d) and pos.is_cuda
+            and keys.is_cuda and values.is_cuda):
+        out = _ext().cached_layer(h, x, packed_weight(w), b, heads, keys, values, pos, rows, order,
+                                  *args)
+        return out[0] if norm is None else (out[0], out[1])
+    q, k, v = (t.reshape(n, heads, d // heads) for t in linear(h, w, b).chunk(3, -1))
+    a = decode_attention_append(q, k, v, keys, values, pos, rows, order=order)
+    return attention_tail(layer, a.reshape(n, d), x, norm)
+
+
 def attention_tail(layer, att: torch.Tensor, x: torch.Tensor, norm: nn.Module | None = None):
     """The rest of a pre-norm encoder layer after its attention (python/cugo_seq50.py:
     317-322): x1 = x + out_proj(att), then feed_forward(layer, norm2(x1), x1, norm).  One
     HIP launch (`out_proj_ffn`: neither x1 nor norm2(x1) leaves the chip) for the d = 256
     bf16 layer `feed_forward` fuses with a biased out_proj and an affine bf16 norm2;
     linear_add_norm and feed_forward otherwise, which give the same bits."""
-    op, n2 = layer.self_attn.out_proj, layer.norm2
-    if (_fits_ffn(layer, att, x, norm) and _fits_linear(att, op.weight, op.bias)
-            and tuple(op.weight.shape) == (256, 256) and op.bias is not None
-            and isinstance(n2, nn.LayerNorm) and n2.weight is not None and n2.bias is not None
-            and n2.weight.dtype == torch.bfloat16 and n2.bias.dtype == torch.bfloat16
-            and tuple(n2.normalized_shape) == (256,)):
-        l1, l2 = layer.linear1, layer.linear2
-        out = _ext().out_proj_ffn(att, x, packed_weight(op.weight), op.bias.detach(),
-                                  n2.weight.detach(), n2.bias.detach(), n2.eps,
-                                  packed_weight(l1.weight), l1.bias.detach(),
-                                  packed_weight(l2.weight), l2.bias.detach(),
-                                  None if norm is None else norm.weight.detach(),
-                                  None if norm is None else norm.bias.detach(),
-                                  1e-5 if norm is None else norm.eps)
+    args = _tail_args(layer, att, x, norm)
+    if args is not None:
+        out = _ext().out_proj_ffn(att, x, *args)
         return out[0] if norm is None else (out[0], out[1])
-    x, h = linear_add_norm(att, op.weight, op.bias, x, n2)
+    op = layer.self_attn.out_proj
+    x, h = linear_add_norm(att, op.weight, op.bias, x, layer.norm2)
     return feed_forward(layer, h, x, norm)
 
 
@@ -249,7 +282,6 @@ def cached_step(model: nn.Module, cache, x: torch.Tensor, slots: int | None = No
     launch."""
     n, d = x.shape
     heads = cache.heads
-    dh = d // heads
     t = cache.slots if slots is None else min(slots, cache.slots)
     row_ids = cache.row_ids if rows is None else rows
     if pos is None:
@@ -262,15 +294,10 @@ def cached_step(model: nn.Module, cache, x: torch.Tensor, slots: int | None = No
     layers = model.encoder.layers
     x, h = add_norm(x, None, layers[0].norm1)
     for i, layer in enumerate(layers):
-        attn = layer.self_attn
-        q, k, v = linear(h, attn.in_proj_weight, attn.in_proj_bias).chunk(3, -1)
-        a = decode_attention_append(q.reshape(n, heads, dh), k.reshape(n, heads, dh),
-                                    v.reshape(n, heads, dh), cache.k[i], cache.v[i], pos,
-                                    row_ids, order=order)
-        if i + 1 < len(layers):
-            x, h = attention_tail(layer, a.reshape(n, d), x, layers[i + 1].norm1)
-        else:
-            x = attention_tail(layer, a.reshape(n, d), x)
+        last = i + 1 == len(layers)
+        out = _layer(layer, h, x, heads, cache.k[i], cache.v[i], pos, row_ids, order,
+                     None if last else layers[i + 1].norm1)
+        x, h = (out, None) if last else out
     return x
 
 
