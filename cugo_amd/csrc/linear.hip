@@ -32,7 +32,9 @@
 //     a quarter-wave (stored from the accumulator layout, a quarter-wave would write 8
 //     bytes into each of 16 rows).
 // Workgroup ids are remapped so that consecutive tiles run on one XCD (the dispatcher
-// deals workgroups to the 8 XCDs in turn), keeping a row panel's reads in one L2.
+// deals workgroups to the 8 XCDs in turn), keeping a row panel's reads in one L2, for any
+// number of them (only for multiples of 8 at first: 15,000 x 768 x 256 17.4 -> 13.0 us, 9,000
+// rows 12.0 -> 10.8, 3,000 rows 6.6 -> 5.3).
 //
 // Arithmetic: bf16 operands, fp32 accumulation in K order; partial rows and columns are
 // clamped on load and masked on store.
@@ -152,7 +154,10 @@ __global__ __launch_bounds__(64 * WR * WC) void linear_kernel(Args a) {
   const int wr = wave / WC, wc = wave % WC;
   int bid = blockIdx.x;
   const int nb = gridDim.x;
-  if ((nb & 7) == 0) bid = (bid & 7) * (nb >> 3) + (bid >> 3);
+  {  // XCD x of 8 takes the x-th run of tiles, one tile longer on the first nb % 8 XCDs
+    const int x = bid & 7, q = nb >> 3, r = nb & 7;
+    bid = x * q + min(x, r) + (bid >> 3);
+  }
   const int rb = bid / a.col_blocks;
   const int m0 = rb * BM;
   const int nb0 = (bid - rb * a.col_blocks) * BN;  // the workgroup's first column
