@@ -77,25 +77,31 @@ PACKED_FP32 = re.compile(r"\bv_pk_(add|mul|fma)_f32\b")
 BUNDLE_MAGIC = b"__CLANG_OFFLOAD_BUNDLE__"
 
 
+def code_objects(lib: Path, tmp: Path) -> list[Path]:
+    """The gfx950 code objects in `lib`'s .hip_fatbin section (one offload bundle per source
+    file), unpacked into the folder `tmp`."""
+    fatbin = tmp / "fatbin"
+    _run(["objcopy", "--dump-section", f".hip_fatbin={fatbin}", str(lib), str(tmp / "copy")])
+    data = fatbin.read_bytes()
+    starts = [m.start() for m in re.finditer(re.escape(BUNDLE_MAGIC), data)]
+    objs = []
+    for k, begin in enumerate(starts):
+        end = starts[k + 1] if k + 1 < len(starts) else len(data)
+        part, obj = tmp / f"b{k}", tmp / f"b{k}.co"
+        part.write_bytes(data[begin:end])
+        _run([str(LLVM_BIN / "clang-offload-bundler"), "--type=o",
+              f"--targets=hipv4-amdgcn-amd-amdhsa--{ARCH}", f"--input={part}",
+              f"--output={obj}", "--unbundle"])
+        objs.append(obj)
+    return objs
+
+
 def device_disassembly(lib: Path) -> str:
-    """The gfx950 disassembly of every code object in `lib`'s .hip_fatbin section (one
-    offload bundle per source file, concatenated)."""
+    """The disassembly of every code object in `lib`, concatenated."""
     with tempfile.TemporaryDirectory() as tmp:
-        fatbin = Path(tmp) / "fatbin"
-        _run(["objcopy", "--dump-section", f".hip_fatbin={fatbin}", str(lib)])
-        data = fatbin.read_bytes()
-        starts = [m.start() for m in re.finditer(re.escape(BUNDLE_MAGIC), data)]
-        text = []
-        for k, begin in enumerate(starts):
-            end = starts[k + 1] if k + 1 < len(starts) else len(data)
-            part, obj = Path(tmp) / f"b{k}", Path(tmp) / f"b{k}.co"
-            part.write_bytes(data[begin:end])
-            _run([str(LLVM_BIN / "clang-offload-bundler"), "--type=o",
-                  f"--targets=hipv4-amdgcn-amd-amdhsa--{ARCH}", f"--input={part}",
-                  f"--output={obj}", "--unbundle"])
-            text.append(subprocess.run([str(LLVM_BIN / "llvm-objdump"), "-d", str(obj)],
-                                       check=True, capture_output=True, text=True).stdout)
-        return "\n".join(text)
+        return "\n".join(subprocess.run([str(LLVM_BIN / "llvm-objdump"), "-d", str(obj)],
+                                        check=True, capture_output=True, text=True).stdout
+                         for obj in code_objects(lib, Path(tmp)))
 
 
 def check_no_packed_fp32(lib: Path) -> None:
