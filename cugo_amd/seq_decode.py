@@ -169,10 +169,12 @@ def _ffn_args(layer, h: torch.Tensor, x: torch.Tensor, norm: nn.Module | None) -
             and x.shape == h.shape and is_exact_gelu(layer.activation)):
         return None
     l1, l2 = layer.linear1, layer.linear2  # each parameter once: a module's lookup is slow
-    w1, b1, w2, b2 = l1.weight, l1.bias, l2.weight, l2.bias
+    w1, w2 = l1.weight, l2.weight
     if not (w1.shape == (1024, 256) and w2.shape == (256, 1024) and w1.dtype == bf16
-            and w2.dtype == bf16 and b1 is not None and b2 is not None and b1.dtype == bf16
-            and b2.dtype == bf16):
+            and w2.dtype == bf16):
+        return None
+    b1, b2 = l1.bias, l2.bias
+    if b1 is None or b2 is None or b1.dtype != bf16 or b2.dtype != bf16:
         return None
     if norm is None:
         return w1, b1, w2, b2, None, None, 1e-5
@@ -208,8 +210,10 @@ def _tail_args(layer, att: torch.Tensor, x: torch.Tensor, norm: nn.Module | None
     """`out_proj_ffn`'s arguments from wo_packed to eps, if it takes the layer: `ffn`'s with a
     biased out_proj and an affine bf16 norm2."""
     args = _ffn_args(layer, att, x, norm)
+    if args is None:
+        return None
     op, n2 = layer.self_attn.out_proj, layer.norm2
-    if args is None or not isinstance(n2, nn.LayerNorm):
+    if not isinstance(n2, nn.LayerNorm):
         return None
     wo, bo, w, b = op.weight, op.bias, n2.weight, n2.bias
     bf16 = torch.bfloat16
@@ -240,7 +244,7 @@ def _layer(layer, h: torch.Tensor, x: torch.Tensor, heads: int, keys: torch.Tens
         return out[0] if norm is None else (out[0], out[1])
     q, k, v = (t.reshape(n, heads, d // heads) for t in linear(h, w, b).chunk(3, -1))
     a = decode_attention_append(q, k, v, keys, values, pos, rows, order=order)
-    return attention_tail(layer, a.reshape(n, d), x, norm)
+    return _tail(layer, a.reshape(n, d), x, norm, args)
 
 
 def attention_tail(layer, att: torch.Tensor, x: torch.Tensor, norm: nn.Module | None = None):
@@ -249,7 +253,11 @@ def attention_tail(layer, att: torch.Tensor, x: torch.Tensor, norm: nn.Module | 
     HIP launch (`out_proj_ffn`: neither x1 nor norm2(x1) leaves the chip) for the d = 256
     bf16 layer `feed_forward` fuses with a biased out_proj and an affine bf16 norm2;
     linear_add_norm and feed_forward otherwise, which give the same bits."""
-    args = _tail_args(layer, att, x, norm)
+    return _tail(layer, att, x, norm, _tail_args(layer, att, x, norm))
+
+
+def _tail(layer, att: torch.Tensor, x: torch.Tensor, norm: nn.Module | None, args: tuple | None):
+    """attention_tail, given _tail_args."""
     if args is not None:
         out = _ext().out_proj_ffn(att, x, *args)
         return out[0] if norm is None else (out[0], out[1])
