@@ -15,24 +15,19 @@
 
 using namespace cugo_amd;
 
+// postchance50.h:509-539 as it stands: the probe, then the apply on a copy that is kept only
+// on success.
 static u8 continue_plain(Env& e, bool& committed) {
   committed = false;
   Pending p = pending_of(e);
-  Env staged;
   Action a = p.action;
-  if (p.sel_pi != 0) {
-    a.pisel = p.sel_pi;
-    const Probe probe = probe_postchance_per_kind(e, p, staged);
-    if (probe.status != kOk) return probe.status;
-    if (probe.decision != kDecNone) return kOk;
-  }
+  if (p.sel_pi != 0) a.pisel = p.sel_pi;
+  Env staged;
+  const Probe probe = probe_postchance_per_kind(e, p, staged);
+  if (probe.status != kOk) return probe.status;
+  if (probe.decision != kDecNone) return kOk;
   Env applied = e;
   const u8 s = apply_action(applied, a);
-  if (s != kOk && p.sel_pi == 0) {
-    const Probe probe = probe_postchance_per_kind(e, p, staged);
-    if (probe.status != kOk) return probe.status;
-    if (probe.decision != kDecNone) return kOk;
-  }
   if (s != kOk) return s;
   e = applied;
   p.action = a;
@@ -48,7 +43,7 @@ static u16 random_legal(const Mask3& m, std::mt19937_64& g) {
   if (c == 0) return kInvalidAction16;
   u32 r = (u32)(g() % c);
   for (u32 i = 0; i < 3; ++i) {
-    if (r < popc(w[i])) return (u16)(64 * i + select_rank(w[i], r));
+    if (r < popc(w[i])) return (u16)(64 * i + select_rank_in(w[i], r));
     r -= popc(w[i]);
   }
   return kInvalidAction16;
