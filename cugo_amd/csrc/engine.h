@@ -136,10 +136,6 @@ CG_HD u8 select_rank_in(u64 mask, u32 rank) {
   if (rank >= c) { rank -= c; w >>= 2; pos += 2; }
   return (u8)(pos + (rank >= (w & 1u) ? 1u : 0u));
 }
-// The same for any rank: kNoCard where no such bit is set.
-CG_HD u8 select_rank(u64 mask, u32 rank) {
-  return rank >= popc(mask) ? kNoCard : select_rank_in(mask, rank);
-}
 
 // ------------------------------------------------------------ month nibbles ----
 // A card mask holds month m in bits 4m..4m+3, so per-month questions are nibble-parallel
@@ -493,7 +489,7 @@ CG_HD void finish_resolved_turn(Env& e) {  // turn50.h:409-416
 CG_HD Resolve resolve_turn(Env& e, u8 played_choice, u8 drawn_choice) {
   Resolve r{kResWrongPhase, 0, 0, 0, 0, 0};
   if (e.phase != kPhaseResolve) return r;
-  Env& n = e;  // in place: the caller's copy is the transaction
+  Env& n = e;  // in place: a failure leaves e partly changed, and reload() restores it
   const u8 played = n.pplayed, drawn = n.pdrawn;
   const u64 pm = floor_matches(n, played);
   const u32 pmc = popc(pm);
@@ -707,7 +703,7 @@ CG_HD PiResult apply_pi_steal(Env& e, u32 thief, u8 requested, u64 selection) {
 
 // pi_transfer.h:234-255: resolve, then steal (on failure the caller discards `e`).
 CG_HD Resolve resolve_turn_with_pi(Env& e, u8 pchoice, u8 dchoice, u64 sel, PiResult& pt) {
-  Env& n = e;  // in place: the caller's copy is the transaction
+  Env& n = e;  // in place: a failure leaves e partly changed, and reload() restores it
   const u8 thief = e.actor;
   const Resolve r = resolve_turn(n, pchoice, dchoice);
   pt = PiResult{kPiOk, 0, 0, 0};
@@ -719,7 +715,7 @@ CG_HD Resolve resolve_turn_with_pi(Env& e, u8 pchoice, u8 dchoice, u64 sel, PiRe
 
 // pi_transfer.h:274-294
 CG_HD u8 play_bonus_with_pi(Env& e, u8 bonus, u64 sel, PiResult& pt, u8& replacement) {
-  Env& n = e;  // in place: the caller's copy is the transaction
+  Env& n = e;  // in place: a failure leaves e partly changed, and reload() restores it
   const u8 thief = e.actor;
   u8 steal;
   const u8 s = play_bonus_for_turn(n, bonus, steal, replacement);
@@ -814,7 +810,7 @@ CG_HD Resolve resolve_game_turn(Env& e, u8 pchoice, u8 dchoice, u64 sel, PiResul
   pt = PiResult{kPiOk, 0, 0, 0};
   if (game_finished(e) || has_pending_choice(e)) return resolve_error(kResWrongPhase);
   const u8 completed = e.actor;
-  Env& n = e;  // in place: the caller's copy is the transaction
+  Env& n = e;  // in place: a failure leaves e partly changed, and reload() restores it
   const Resolve r = resolve_turn_with_pi(n, pchoice, dchoice, sel, pt);
   if (r.status != kResOk || pt.status != kPiOk) return r;
   finish_turn_game(n, completed);
@@ -911,7 +907,7 @@ CG_HD u8 begin_shake(Env& e, u8 card, u16 shake_months) {
   const u16 mb = month_bit(card);
   const u64 hand = active_hand(e);
   if ((shake_months & mb) == 0 || (hand & bit(card)) == 0) return kSpNotLegal;
-  Env& n = e;  // in place: the caller's copy is the transaction
+  Env& n = e;  // in place: a failure leaves e partly changed, and reload() restores it
   const bool four = popc(hand & month_cards(card >> 2)) == 4;
   if (four) { if (n.actor == 0) n.sh4_0 |= mb; else n.sh4_1 |= mb; }
   else { if (n.actor == 0) n.shaken0 |= mb; else n.shaken1 |= mb; }
@@ -933,7 +929,7 @@ CG_HD u8 capture_special(Env& e, u8 month, bool grenade, u8 choice, u64 sel, PiR
   const u16 mb = (u16)(1u << month);
   const u16 legal = grenade ? legal_grenade_months(e) : legal_bomb_months(e);
   if ((legal & mb) == 0) return kSpNotLegal;
-  Env& n = e;  // in place: the caller's copy is the transaction
+  Env& n = e;  // in place: a failure leaves e partly changed, and reload() restores it
   const u8 actor = n.actor;
   const u64 hand = hand_of(n, actor);
   const u64 hc = hand & month_cards(month);
@@ -959,7 +955,7 @@ CG_HD u8 play_bomb_credit(Env& e, u8 choice, u64 sel, PiResult& pt) {
   if (!special_ready(e)) return kSpWrongPhase;
   const u8 actor = e.actor;
   if (!cred_of(e, actor)) return kSpNotLegal;
-  Env& n = e;  // in place: the caller's copy is the transaction
+  Env& n = e;  // in place: a failure leaves e partly changed, and reload() restores it
   set_cred(n, actor, (u8)(cred_of(n, actor) - 1u));
   const DrawOnly d = draw_only_special(n, choice);
   if (d.status != kSpOk) return d.status;
@@ -1127,7 +1123,7 @@ CG_HD u8 play_bonus_terminal(Env& e, u8 bonus, u64 sel, PiResult& pt) {
   pt = PiResult{kPiOk, 0, 0, 0};
   if (terminal_finished(e) || has_ct_choice(e)) return kTurnWrongPhase;
   if (game_finished(e) || has_pending_choice(e)) return kTurnWrongPhase;  // game50.h:263-267
-  Env& n = e;  // in place: the caller's copy is the transaction
+  Env& n = e;  // in place: a failure leaves e partly changed, and reload() restores it
   const u8 actor = n.actor;
   const u16 before = chongtong_months(active_hand(n));
   u8 replacement;
@@ -1143,7 +1139,7 @@ CG_HD u8 play_bonus_terminal(Env& e, u8 bonus, u64 sel, PiResult& pt) {
 CG_HD Resolve resolve_terminal_turn(Env& e, u8 pchoice, u8 dchoice, u64 sel, PiResult& pt) {
   pt = PiResult{kPiOk, 0, 0, 0};
   if (terminal_finished(e) || has_ct_choice(e)) return resolve_error(kResWrongPhase);
-  Env& n = e;  // in place: the caller's copy is the transaction
+  Env& n = e;  // in place: a failure leaves e partly changed, and reload() restores it
   const u8 actor = n.actor;
   const u64 before = cap_of(n, actor);
   const Resolve r = resolve_game_turn(n, pchoice, dchoice, sel, pt);
@@ -1158,7 +1154,7 @@ CG_HD Resolve resolve_terminal_turn(Env& e, u8 pchoice, u8 dchoice, u64 sel, PiR
 // terminal50.h:505-530 for bomb/grenade/bomb-credit (shake handled by its caller).
 CG_HD u8 apply_terminal_special(Env& e, u8 kind, u8 month, u8 choice, u64 sel) {
   if (terminal_finished(e) || has_ct_choice(e)) return kSpWrongPhase;
-  Env& n = e;  // in place: the caller's copy is the transaction
+  Env& n = e;  // in place: a failure leaves e partly changed, and reload() restores it
   const u8 actor = n.actor;
   const u64 before = cap_of(n, actor);
   PiResult pt;
@@ -1178,7 +1174,7 @@ CG_HD u8 apply_terminal_shake(Env& e, u8 card) {  // terminal50.h:505-530, kShak
 
 CG_HD u8 apply_terminal_gukjin(Env& e, bool as_pi) {  // terminal50.h:532-544
   if (terminal_finished(e) || has_ct_choice(e)) return 2;
-  Env& n = e;  // in place: the caller's copy is the transaction
+  Env& n = e;  // in place: a failure leaves e partly changed, and reload() restores it
   const u8 s = apply_gukjin_decision(n, as_pi);
   if (s != 0) return s;
   sync_game_stop(n);
@@ -1187,7 +1183,7 @@ CG_HD u8 apply_terminal_gukjin(Env& e, bool as_pi) {  // terminal50.h:532-544
 
 CG_HD u8 apply_terminal_go_stop(Env& e, bool stop) {  // terminal50.h:546-559
   if (terminal_finished(e) || has_ct_choice(e)) return 2;
-  Env& n = e;  // in place: the caller's copy is the transaction
+  Env& n = e;  // in place: a failure leaves e partly changed, and reload() restores it
   const u8 s = apply_go_stop(n, stop);
   if (s != 0) return s;
   sync_game_stop(n);
@@ -1323,8 +1319,8 @@ CG_HD bool is_turn_kind(u8 k) {
 //   * the bookkeeping: terminal50.h:456-503 for a played card, 505-530 for a special,
 //     415-454 for a bonus play.
 // The checks run in the composition's order and return its statuses; the state updates
-// are the composition's, in its order.  `n` is the caller's transaction copy: a failure
-// may leave it partly changed.
+// are the composition's, in its order.  `n` is the live state: a failure may leave it partly
+// changed, and the caller (continue_postchance) then puts it back from reload().
 CG_HD u8 apply_turn_action(Env& n, const Action& a) {
   const u8 actor = n.actor;
   const bool bonus = a.kind == kPlayBonus;
@@ -1464,10 +1460,11 @@ CG_HD u8 apply_turn_action(Env& n, const Action& a) {
   return kOk;
 }
 
-// rollout50.h:231-385; the held-card bookkeeping of apply_action50 (391-399) included.
+// rollout50.h:231-385; the held-card bookkeeping of apply_action50 (391-399) included.  In
+// place: after a status other than kOk `e` is partly changed and to be restored by the caller.
 CG_HD u8 apply_action(Env& e, const Action& a) {
   if (terminal_finished(e)) return kGameFinished;
-  Env& n = e;  // in place: the caller's copy is the transaction
+  Env& n = e;  // in place: a failure leaves e partly changed, and reload() restores it
   n.held0 |= n.hand0;
   n.held1 |= n.hand1;
   if (a.kind == kChongtongWin || a.kind == kChongtongContinue) {
@@ -2578,7 +2575,7 @@ struct FeatRow {
 // division's ~10 instructions: multiply by the rounded reciprocal, then one correction with
 // the exact remainder (two FMAs).  A power-of-two scale is the exact multiply that the
 // compiler makes of the division by itself.  Equal to the division for every value below
-// 65,536 and every scale used here (tests/engine_host_check.cpp).
+// 65,536 and every scale used here (tests/engine_step_check.cpp).
 template <u32 kScale>
 CG_HD float quotient(u32 value) {
   if constexpr ((kScale & (kScale - 1u)) == 0u) {

@@ -2,8 +2,8 @@
 // Built and run by tests/test_cpu_engine_host.py (host code only; no GPU):
 //  1. feature_record + the GPU writer's decode (nibble -> 0/1.0f patterns, OR the dense
 //     dword or the zero pad) == feature_at for every one of the 720 features;
-//  2. hangame_steal_selection (six mask passes) == the card-by-card loop of
-//     pi_transfer.h:90-110;
+//  2. hangame_steal_selection (the first key's lowest card, a card a pass) == the card-by-card
+//     loop of pi_transfer.h:90-110;
 //  3. special_months == legal_special_months (special50.h:71-95) for bombs, grenades and
 //     shakes;
 //  4. apply_turn_action (the six turn-taking kinds as one transition) == the per-kind
@@ -126,7 +126,7 @@ static int check_special_months(std::mt19937_64& g) {
 // Any set bit of m, or kNoCard.
 static u8 any_bit(u64 m, std::mt19937_64& g) {
   const u32 c = (u32)__builtin_popcountll(m);
-  return c == 0 ? kNoCard : select_rank(m, (u32)(g() % c));
+  return c == 0 ? kNoCard : select_rank_in(m, (u32)(g() % c));
 }
 
 static int check_turn_actions(std::mt19937_64& g) {
@@ -198,7 +198,7 @@ static int check_turn_actions(std::mt19937_64& g) {
       u16 act = 0;
       for (u32 i = 0; i < 3; ++i) {
         const u32 ci = (u32)__builtin_popcountll(w[i]);
-        if (r < ci) { act = (u16)(64 * i + select_rank(w[i], r)); break; }
+        if (r < ci) { act = (u16)(64 * i + select_rank_in(w[i], r)); break; }
         r -= ci;
       }
       torch_step(e, act);
