@@ -127,12 +127,13 @@ HEADERS = (CSRC / "engine.h", REPO / "include" / "cugo_hip.h")
 
 def build_library(force: bool = True) -> Path:
     """Compiles each source to an object under _build/ (in parallel; with force=False only
-    those older than their source or a shared header), then links the library."""
+    those older than their source, a shared header or this file, which holds the flags), then
+    links the library."""
     generate_stop_bits(force=force)
     out = PKG / "libcugo_hip.so"
     objdir = PKG / "_build"
     objdir.mkdir(exist_ok=True)
-    shared = [*HEADERS, CSRC / "stop_bits.inc"]
+    shared = [*HEADERS, CSRC / "stop_bits.inc", Path(__file__)]
     procs, objs = [], []
     for name in SOURCES:
         src, obj = CSRC / name, objdir / (name + ".o")
