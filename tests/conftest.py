@@ -38,16 +38,3 @@ def ext():
 
 def announce(name: str) -> None:
     print(f"[case] {name}", flush=True)
-
-
-def poison_free_memory() -> None:
-    """Fills the GPU memory that torch's allocator hands out next with 0xA5 bytes, so that an
-    element that a kernel does not write differs from what an earlier call left there."""
-    import torch
-
-    torch.cuda.empty_cache()
-    held = [torch.full((2 << 30,), 0xA5, dtype=torch.uint8, device="cuda")]
-    for k in range(9, 21):  # the allocator keeps sizes up to 1 MiB apart, in pieces
-        held += [torch.full((1 << k,), 0xA5, dtype=torch.uint8, device="cuda") for _ in range(32)]
-    del held
-    assert bool((torch.empty(1 << 24, dtype=torch.uint8, device="cuda") == 0xA5).all())

@@ -1,13 +1,12 @@
 """The MLP actor's rows a tile, chosen by batch, change no row's result: a batch at each edge
-of the choice (and one past it, and partial last tiles) gives the first rows of what a batch
-of 128-row tiles gives, bit for bit, over the depths, widths and input types it takes."""
+of the choice (and one past it, and partial last tiles) gives the last rows of what a batch
+of 128-row tiles gives, bit for bit, over the depths, widths and input types it takes.  (The last
+ones, so that each batch has other rows: outputs may lie where an earlier batch's lay.)"""
 
 from __future__ import annotations
 
 import pytest
 import torch
-
-from tests.conftest import poison_free_memory
 
 pytestmark = pytest.mark.gpu
 
@@ -43,10 +42,9 @@ def test_actor_tiles_give_the_same_rows(ext, blocks, features, actions, dtype, s
         want_l, want_v = mlp_forward(ext, packed, x)
         assert torch.isfinite(want_l.float()).all() and torch.isfinite(want_v).all()
         for n in sizes:
-            part = x[:n].contiguous()
+            part = x[BIG - n:].contiguous()
             copy = torch.full((n, features), float("nan"), dtype=torch.bfloat16, device=DEV)
-            poison_free_memory()  # the same rows were in the outputs of the batch before
             got_l, got_v = mlp_forward(ext, packed, part, copy)
-            assert torch.equal(got_l, want_l[:n]), n
-            assert torch.equal(got_v, want_v[:n]), n
+            assert torch.equal(got_l, want_l[BIG - n:]), n
+            assert torch.equal(got_v, want_v[BIG - n:]), n
             assert torch.equal(copy, part.to(torch.bfloat16)), n
