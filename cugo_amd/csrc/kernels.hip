@@ -465,11 +465,11 @@ __device__ inline i64 spare_row(const AutoReset& ar, i64 i, u32 gen) {
 // kMode: 0 = step (contiguous, in place), 1 = step_indexed (gather/scatter in place),
 // 3 = step with the auto-reset above (contiguous, in place); branch_indexed has its own
 // kernel below.
-// kThreads = 128: two waves per tile of 64 games, both stage the rows in and out and
-// wave 0 runs the games (one per lane).  At ~250 VGPRs two waves fit per SIMD, so this
-// is the shape while every tile of the grid is resident at once (up to four per CU);
-// a larger grid queues tiles, and then one wave per tile (kThreads = 64) keeps twice as
-// many games computing per CU.
+// Games a tile: see step_rows.  kStepThreads = 128 (tiles of 32 and 64 games): two waves per
+// tile, both stage the rows in and out and wave 0 runs the games (one per lane).  At 165-222
+// VGPRs two or three waves fit per SIMD, so this is the shape while every tile of the grid is
+// resident at once (up to four per CU); a larger grid queues tiles, and then one wave per tile
+// (kStepThreads = 64) keeps twice as many games computing per CU.
 template <int kMode, bool kEvents, int kStepThreads, int kRows = kTile>
 __global__ __launch_bounds__(kStepThreads) void step_kernel(u64* states, i64 env_count, const i64* ids,
                                                      const i64* actions, i64 n,
@@ -575,7 +575,8 @@ __global__ __launch_bounds__(kStepThreads) void step_kernel(u64* states, i64 env
 // broadcasts from L2), steps it in registers, and the wave's 64 child rows go out through
 // LDS as contiguous blocks.  An action that fails reads its parent again, so the
 // transition keeps one state in registers: 168 VGPRs, three waves per SIMD (with a second
-// state kept they were 198 and two waves; 262,144 children 31.7 -> 27.4 us).  Capping
+// state kept they were 198 and two waves; 262,144 children 31.7 -> 27.4 us), with 8 bytes
+// spilled a lane on 64-row tiles.  Capping
 // registers for four waves spills ~150 bytes a lane; staging the parents through LDS as
 // well, as the other step kernels do, measured 1.13x slower when two waves fit.
 // kRows children a wavefront: see branch_rows().
@@ -1476,10 +1477,22 @@ inline int device_cus() {
 //                       256: 250 / 252 / 231 / 209 / 196 / 177 / 152
 //                       1,024: 260 / 267 / 241 / 216 / 195 / 250 / 305
 //                       4,096: 259 / 284 / 251 / 294 / 392         32,768: 278 / 246 / 287
-// Grids of one-wavefront workgroups between one and about five a CU run slower than smaller
+// Grids of one-wavefront workgroups between one and about four a CU run slower than smaller
 // and larger ones (the same loop of plain FMAs takes 11 % longer at 512 wavefronts than
 // at 256 or 1,024), which is why the step's line for 4,096 rows is 16 games and the one
-// for 8,192 is 4.
+// for 8,192 is 4.  On both sides of that line (graphs of 4 launches):
+//   step with auto-reset (64 / 32 / 16 / 8 / 4)
+//                       3,000: 20.4 / 19.6 / 18.4 / 19.1 / 19.5    4,096: 20.2 / 19.8 / 18.4 / 19.1 / 20.8
+//                       4,500: 20.3 / 19.7 / 19.8 / 20.7 / 17.8    5,200: 20.3 / 19.6 / 21.3 / 21.3 / 17.1
+//                       7,000: 20.4 / 19.7 / 21.5 / 22.5 / 17.0    8,192: 20.1 / 19.8 / 21.8 / 23.3 / 17.3
+//                       10,000: 20.2 / 19.2 / 18.9 / 18.8 / 24.7
+//   step_observe (64 / 32 / 16 / 4)
+//                       2,048: 42.8 / 33.3 / 28.1 / 24.2           4,096: 42.1 / 33.5 / 28.3 / 27.3
+//                       4,500: 42.4 / 33.7 / 30.7 / 26.7           7,000: 42.6 / 34.2 / 32.4 / 25.8
+//                       10,000: 42.9 / 34.9 / 30.7 / 37.5
+//   rollout_canonical (64 / 32 / 16 / 8 / 4), where 64 games are taken from 4,097 to 16,384
+//                       4,500: 276 / 287 / 334 / 373 / 316         8,192: 271 / 286 / 351 / 447 / 262
+//                       10,000: 273 / 292 / 291 / 279 / 302        16,384: 271 / 276 / 247 / 289 / 477
 inline int play_rows(int64_t n) {
   return n <= 4096 ? 4 : n <= 8192 ? 8 : n <= 16384 ? 16 : n <= 32768 ? 32 : kTile;
 }

@@ -1202,8 +1202,8 @@ std::vector<torch::Tensor> out_proj_ffn(torch::Tensor att, torch::Tensor x,
 // out_proj_ffn's arguments from wo_packed to eps) -> as out_proj_ffn: a pre-norm layer of one
 // token a row (python/cugo_seq50.py:310-322), h = norm1(x): linear, decode_attention_append
 // on its q, k and v in place, out_proj_ffn.  One call instead of three with the views between
-// them: below ~5,000 rows the host's work, not the launches, is a layer's time (500 rows 51.4 ->
-// 35.2 us a layer, with the fewer parameter lookups of its caller).
+// them: below ~5,000 rows the host's work, not the launches, is an eager layer's time (500 rows
+// 51.3 -> 36.2 us a layer, with the fewer parameter lookups of its caller).
 std::vector<torch::Tensor> cached_layer(
     torch::Tensor h, torch::Tensor x, torch::Tensor in_packed, c10::optional<torch::Tensor> in_bias,
     int64_t heads, torch::Tensor keys, torch::Tensor values, torch::Tensor pos,
