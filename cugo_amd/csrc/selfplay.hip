@@ -374,7 +374,9 @@ struct PhiloxNoise {
 // -1e30 can win or be the maximum); any other takes all the actions.  The rows are counted
 // first, in the lanes and by four DPP adds, so that the others pay little more than that count.
 // 65,536 bf16 rows, us with all the actions always / packed as they are counted / counted
-// first: 10 legal actions 27.7 / 19.0 / 17.4, 40 legal actions 27.7 / 35.8 / 29.0.
+// first: 10 legal actions 27.7 / 18.1 / 16.5, 40 legal actions 27.7 / 35.3 / 28.1.  The legal
+// actions are one word of bits and the loads' addresses 32-bit offsets, so that the registers
+// (64 at most) hold a whole chip's rows at once.
 // The exponentials go back through LDS to the lanes that hold the actions, which sum them in
 // the order of the other way: the same bits.
 constexpr int kGumbelLanes = 16;
@@ -382,69 +384,105 @@ constexpr int kGumbelPer = 12;  // up to 192 actions
 constexpr int kGumbelPacked = 2 * kGumbelLanes;
 static_assert(kGumbelPer == 12, "a Philox lane draws three blocks of four uniforms");
 
-template <class T, int kNoise>
-__global__ __launch_bounds__(256) void gumbel_rows_kernel(
+// With Philox, 512 threads a workgroup where all workgroups are resident at once and share the
+// CUs evenly: waves that end in their own time leave the dispatcher in a state in which it
+// puts two computing waves of the launch behind (step_observe's, one a SIMD) on one SIMD, at
+// about 10 of the 1,024 SIMDs, and that launch waits for them.  Workgroups of 512 leave none.
+// Sampler and engine step, us with 512 / 256 threads: 32,768 rows 52.7 / 53.4-54.2, 24,576
+// 50.1 / 50.4, 16,384 41.4 / 41.3, 8,192 33.5 / 33.5; where the last round of workgroups
+// leaves CUs idle the larger ones lose: 12,288 rows 40.4 / 39.4, 20,000 49.3 / 48.4, 28,000
+// 54.8 / 51.6, and 4,096 rows, which leave CUs empty, the sampler alone 4.9 / 4.4.
+inline bool gumbel_wide(i64 n) {
+  constexpr i64 kRows = 512 / kGumbelLanes;
+  thread_local int device = -1, cus = 256;
+  int now = 0;
+  if (hipGetDevice(&now) != hipSuccess) return false;
+  if (now != device) {
+    int count = 0;
+    cus = hipDeviceGetAttribute(&count, hipDeviceAttributeMultiprocessorCount, now) ==
+                      hipSuccess && count > 0 ? count : 256;
+    device = now;
+  }
+  const i64 groups = (n + kRows - 1) / kRows;
+  const i64 rounds = (groups + cus - 1) / cus;  // workgroups a CU, four of which are resident
+  return rounds <= 4 && groups * 16 >= rounds * cus * 15;
+}
+
+template <class T, int kNoise, int kThreads = 256>
+__global__ __launch_bounds__(kThreads) void gumbel_rows_kernel(
     const typename T::storage* logits, const uint8_t* legal, const float* u, i64 n,
     int actions_count, i64* actions, float* logp, PhiloxNoise px) {
   const int j = threadIdx.x & (kGumbelLanes - 1);
-  const i64 r = (i64)blockIdx.x * (256 / kGumbelLanes) + (threadIdx.x / kGumbelLanes);
+  const i64 r = (i64)blockIdx.x * (kThreads / kGumbelLanes) + (threadIdx.x / kGumbelLanes);
   const bool row_ok = r < n;
   // Every load is unconditional, at an index clamped into the arrays (a lane past the
   // last row or action reads an element that exists and ignores it), so all of a lane's
   // loads are in flight together instead of each waiting on the legal byte before it.
   const i64 rr = row_ok ? r : n - 1;
-  const typename T::storage* lr = logits + rr * actions_count;
-  const uint8_t* gr = legal + rr * actions_count;
-  const float* ur = kNoise == 1 ? u + rr * actions_count : nullptr;
+  // The workgroup's rows start at a scalar address and a lane keeps 32-bit offsets from it:
+  // 64-bit addresses of every load would hold twice the registers.
+  const i64 r0 = (i64)blockIdx.x * (kThreads / kGumbelLanes);
+  const typename T::storage* lr = logits + r0 * actions_count;
+  const uint8_t* gr = legal + r0 * actions_count;
+  const float* ur = kNoise == 1 ? u + r0 * actions_count : nullptr;
+  const uint32_t row_at = (uint32_t)(rr - r0) * (uint32_t)actions_count;
+  auto at_offset = [](auto* p, uint32_t i) {
+    return *reinterpret_cast<decltype(p)>(reinterpret_cast<const char*>(p) +
+                                          i * (uint32_t)sizeof(*p));
+  };
   uint8_t gb[kGumbelPer];
   typename T::storage lv[kGumbelPer];
-  float uv[kGumbelPer];
+  float uv[kGumbelPer], x[kGumbelPer];
+  uint32_t legal_bits = 0;  // bit k: action j + 16 k is legal (kNoise 2)
 #pragma unroll
   for (int k = 0; k < kGumbelPer; ++k) {
     const int a = j + kGumbelLanes * k;
-    const int ac = a < actions_count ? a : actions_count - 1;
-    gb[k] = gr[ac];
-    lv[k] = lr[ac];
-    uv[k] = kNoise == 1 ? ur[ac] : 0.0f;
+    const uint32_t ac = row_at + (uint32_t)(a < actions_count ? a : actions_count - 1);
+    gb[k] = at_offset(gr, ac);
+    lv[k] = at_offset(lr, ac);
+    uv[k] = kNoise == 1 ? at_offset(ur, ac) : 0.0f;
   }
   if constexpr (kNoise >= 2) {
     const uint32_t epoch = (uint32_t)*px.epoch;
     const uint32_t row_hi = (uint32_t)((uint64_t)rr >> 32) << 8;
     if constexpr (kNoise == 2) {
       __builtin_amdgcn_sched_barrier(0);  // the loads of the logits are not put behind the count
-      int at[kGumbelPer];  // where this lane's legal actions are packed; -1: not legal
-      int count = 0;       // the row's legal actions: a sum over its 16 lanes, one DPP row
 #pragma unroll
       for (int k = 0; k < kGumbelPer; ++k) {
         const int a = j + kGumbelLanes * k;
-        at[k] = row_ok && a < actions_count && gb[k] != 0 ? 0 : -1;
-        count += at[k] + 1;
+        legal_bits |= (uint32_t)(row_ok && a < actions_count && gb[k] != 0) << k;
       }
+      // the row's legal actions: a sum over its 16 lanes, one DPP row
+      int count = __popc(legal_bits);
       count += __builtin_amdgcn_mov_dpp(count, 0x128, 0xf, 0xf, false);  // rotated by 8 lanes
       count += __builtin_amdgcn_mov_dpp(count, 0x124, 0xf, 0xf, false);
       count += __builtin_amdgcn_mov_dpp(count, 0x122, 0xf, 0xf, false);
       count += __builtin_amdgcn_mov_dpp(count, 0x121, 0xf, 0xf, false);
+#pragma unroll
+      for (int k = 0; k < kGumbelPer; ++k) x[k] = T::to_float(lv[k]);
       bool packs = __ballot(count > kGumbelPacked) == 0;
       if (packs) {
         int plain = 1;  // no branches
 #pragma unroll
         for (int k = 0; k < kGumbelPer; ++k)
-          plain &= (int)(at[k] < 0) | (int)(T::to_float(lv[k]) > -1.0e29f);
+          plain &= (int)(~legal_bits >> k & 1u) | (int)(x[k] > -1.0e29f);
         packs = __ballot(plain == 0) == 0;
       }
       if (packs) {
-        __shared__ uint2 packed[256 / kGumbelLanes][kGumbelPacked];  // action, logit
+        __shared__ uint2 packed[kThreads / kGumbelLanes][kGumbelPacked];  // action, logit
         uint2* slots = packed[threadIdx.x / kGumbelLanes];
         const int shift = threadIdx.x & (64 - kGumbelLanes);  // the row's bits of a ballot
         int before = 0;
+        int at[kGumbelPer];  // where this lane's legal actions are packed
 #pragma unroll
         for (int k = 0; k < kGumbelPer; ++k) {
-          const bool legal_a = at[k] >= 0;
+          at[k] = -1;
+          const bool legal_a = (legal_bits >> k & 1u) != 0;
           const uint32_t bits = (uint32_t)(__ballot(legal_a) >> shift) & ((1u << kGumbelLanes) - 1);
           if (legal_a) {
             at[k] = before + __popc(bits & ((1u << j) - 1));
             slots[at[k]] =
-                make_uint2((uint32_t)(j + kGumbelLanes * k), __float_as_uint(T::to_float(lv[k])));
+                make_uint2((uint32_t)(j + kGumbelLanes * k), __float_as_uint(x[k]));
           }
           before += __popc(bits);
         }
@@ -525,8 +563,8 @@ __global__ __launch_bounds__(256) void gumbel_rows_kernel(
   for (int k = 0; k < kGumbelPer; ++k) {
     const int a = j + kGumbelLanes * k;
     const bool in = row_ok && a < actions_count;
-    ok[k] = in && gb[k] != 0;
-    m[k] = ok[k] ? T::to_float(lv[k]) : -1.0e30f;
+    ok[k] = kNoise == 2 ? (legal_bits >> k & 1u) != 0 : in && gb[k] != 0;
+    m[k] = ok[k] ? (kNoise == 2 ? x[k] : T::to_float(lv[k])) : -1.0e30f;
     uc[k] = fmaxf(uv[k], 1.0e-20f);
     if (kNoise == 1) uc[k] = fminf(uc[k], 1.0f);  // Philox's are below 1
   }
@@ -1051,18 +1089,24 @@ int cugo_gumbel_sample_philox(int logits_dtype, const void* logits, const uint8_
   if (n == 0) return 0;
   if (logits_dtype != CUGO_DTYPE_F32 && logits_dtype != CUGO_DTYPE_BF16) return -2;
   const PhiloxNoise px{(uint32_t)seed, (uint32_t)(seed >> 32), offset, epoch, uniforms_out};
-  const unsigned grid = (unsigned)((n + 256 / kGumbelLanes - 1) / (256 / kGumbelLanes));
-#define CUGO_GUMBEL_ROWS(TT, NOISE, PTR)                                            \
-  gumbel_rows_kernel<TT, NOISE><<<grid, 256, 0, stream>>>(                          \
-      (PTR)logits, legal, nullptr, n, (int)actions_count, actions, logp, px)
-  if (logits_dtype == CUGO_DTYPE_F32) {
-    if (uniforms_out) CUGO_GUMBEL_ROWS(F32, 3, const float*);
-    else CUGO_GUMBEL_ROWS(F32, 2, const float*);
+  const auto go = [&](auto kernel, const auto* rows, int threads) {
+    const int per = threads / kGumbelLanes;
+    kernel<<<(unsigned)((n + per - 1) / per), threads, 0, stream>>>(
+        rows, legal, nullptr, n, (int)actions_count, actions, logp, px);
+  };
+  const bool f32 = logits_dtype == CUGO_DTYPE_F32;
+  const float* x32 = static_cast<const float*>(logits);
+  const uint16_t* x16 = static_cast<const uint16_t*>(logits);
+  if (uniforms_out) {
+    if (f32) go(gumbel_rows_kernel<F32, 3>, x32, 256);
+    else go(gumbel_rows_kernel<BF16, 3>, x16, 256);
+  } else if (!gumbel_wide(n)) {
+    if (f32) go(gumbel_rows_kernel<F32, 2>, x32, 256);
+    else go(gumbel_rows_kernel<BF16, 2>, x16, 256);
   } else {
-    if (uniforms_out) CUGO_GUMBEL_ROWS(BF16, 3, const uint16_t*);
-    else CUGO_GUMBEL_ROWS(BF16, 2, const uint16_t*);
+    if (f32) go(gumbel_rows_kernel<F32, 2, 512>, x32, 512);
+    else go(gumbel_rows_kernel<BF16, 2, 512>, x16, 512);
   }
-#undef CUGO_GUMBEL_ROWS
   return (int)hipGetLastError();
 }
 

@@ -25,12 +25,14 @@ def _legal(n, a, counts, g):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("n,a", [(4099, 179), (1, 179), (67, 192), (130, 16), (130, 15), (9, 1)])
+@pytest.mark.parametrize("n,a", [(4099, 179), (1, 179), (67, 192), (130, 16), (130, 15), (9, 1),
+                                 (7681, 179), (8161, 192), (8192, 15), (32767, 179)])
 def test_gumbel_packed_rows(ext, dtype, n, a):
     """Actions and log-probabilities of gumbel_sample_philox, which packs rows of few legal
     actions, against gumbel_sample on the same uniforms, which never does: the same bits, at
     0 to 33 legal actions a row (33 is past the packing), mixed within wavefronts and alike
-    in them, with ties, infinities and the type's lowest value among the logits."""
+    in them, with ties, infinities and the type's lowest value among the logits; the last four
+    sizes are taken by the larger workgroups (a whole last one, one of a single row, odd rows)."""
     g = torch.Generator(device=DEV).manual_seed(n + a)
     epoch = torch.tensor([7], dtype=torch.int64, device=DEV)
     low = torch.finfo(dtype).min
