@@ -274,28 +274,38 @@ CG_HD Score score_captured(u64 cards, bool gukjin_pi) {  // hwatu.h:153-199
 // Register form of the reference TorchEnv50 (torch50.h:108-121): TurnState50
 // (turn50.h:92-115), GameState50 (game50.h:38-48), SpecialGameState50
 // (special50.h:25-32), TerminalGameState50 (terminal50.h:74-102), PostChancePending50
-// (postchance50.h:22-28) and the counters, flattened.  Fields by size, so that there are no
-// holes: a struct copy copies the holes too, and one of 3 or 7 bytes does not become a
-// register.  Two of them lived in LDS through play_kernel's copies, at an address computed
-// from the dispatch packet, which is in host memory: each workgroup's read of it held up the
-// launch (play_random of one step, 131,072 games 137 us with them, 113 without; 33,000 games
-// 61 and 49).
+// (postchance50.h:22-28) and the counters, flattened.  Near the reference's order, with small
+// fields moved into its holes: a struct copy copies the holes too, and one of 3 or 7 bytes does
+// not become a register.  Two of them lived in LDS through play_kernel's copies, at an address
+// computed from the dispatch packet, which is in host memory: each workgroup's read of it held
+// up the launch (play_random of one step, 131,072 games 137 us with them, 113 without; 33,000
+// games 61 and 49).  Sorted by size, which leaves no hole either, the kernels take more
+// registers: branch_kernel 168 and 8 bytes spilled (155 so), canonical_kernel 155 (142),
+// step_observe_kernel 182 (171); us sorted / so: play_random x 32, 3,001 games 313 / 306;
+// 250,000 canonical games 554 / 550; 800,000 children 54.2 / 52.9.
 struct Env {
-  u64 hand0, hand1, floor, stock, cap0, cap1, rng, pend_bonus, mission, tpoints;
-  u64 held0, held1, rev0, rev1, a_pisel, sel_pi;
-  i32 side0;
-  u16 ppuk, owner1, b2ppuk, b3ppuk, turn, neutral, shaken0, shaken1, sh4_0, sh4_1, ct_months;
-  u16 prim, n_primary, n_choice, n_resolve, n_pi, n_bonus, n_special, n_go;
+  u64 hand0, hand1, floor, stock, cap0, cap1, rng, pend_bonus;
+  u16 ppuk, owner1, b2ppuk, b3ppuk, turn;
   u8 actor, phase, pplayed, pdrawn;
-  u8 go0, go1, lgo0, lgo1, dact, winner, gdec;
+  u16 n_go;
+  u64 mission;
+  u16 neutral;
+  u8 go0, go1, lgo0, lgo1, dact, winner, gdec, nagari;
+  u16 shaken0, shaken1;
   u8 bombs0, bombs1, cred0, cred1;
+  u16 sh4_0, sh4_1;
   u8 pcount0, pcount1, streak0, streak1, ct_actor;
+  u16 ct_months;
   u8 twinner, treason;
-  u8 round, mtype, mmult, mm0, mm1;
-  // pending post-chance action (Action50 at 192, rollout50.h:46-52), with a_pisel and sel_pi
-  u8 a_kind, a_card, a_month, a_pmatch, a_dmatch;
-  u8 pactor, pactive;
-  u8 status, done, nagari;
+  u64 tpoints;
+  i32 side0;
+  u8 round, mtype, mmult, mm0, mm1, done;
+  u16 prim, n_primary, n_choice;
+  u64 held0, held1, rev0, rev1;
+  // pending post-chance action (Action50 at 192, rollout50.h:46-52)
+  u8 a_kind, a_card, a_month, a_pmatch, a_dmatch, pactor, pactive, status;
+  u64 a_pisel, sel_pi;
+  u16 n_resolve, n_pi, n_bonus, n_special;
 };
 
 // The 248-byte row as 31 little-endian words; every byte not listed is padding.

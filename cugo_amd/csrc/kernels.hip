@@ -466,7 +466,7 @@ __device__ inline i64 spare_row(const AutoReset& ar, i64 i, u32 gen) {
 // 3 = step with the auto-reset above (contiguous, in place); branch_indexed has its own
 // kernel below.
 // Games a tile: see step_rows.  kStepThreads = 128 (tiles of 32 and 64 games): two waves per
-// tile, both stage the rows in and out and wave 0 runs the games (one per lane).  At 165-222
+// tile, both stage the rows in and out and wave 0 runs the games (one per lane).  At 151-210
 // VGPRs two or three waves fit per SIMD, so this is the shape while every tile of the grid is
 // resident at once (up to four per CU); a larger grid queues tiles, and then one wave per tile
 // (kStepThreads = 64) keeps twice as many games computing per CU.
@@ -574,9 +574,8 @@ __global__ __launch_bounds__(kStepThreads) void step_kernel(u64* states, i64 env
 // global memory (branching children of one root read the same row, so a wave's loads are
 // broadcasts from L2), steps it in registers, and the wave's 64 child rows go out through
 // LDS as contiguous blocks.  An action that fails reads its parent again, so the
-// transition keeps one state in registers: 168 VGPRs, three waves per SIMD (with a second
-// state kept they were 198 and two waves; 262,144 children 31.7 -> 27.4 us), with 8 bytes
-// spilled a lane on 64-row tiles.  Capping
+// transition keeps one state in registers: 155 VGPRs, three waves per SIMD (with a second
+// state kept they were 198 and two waves; 262,144 children 31.7 -> 27.4 us).  Capping
 // registers for four waves spills ~150 bytes a lane; staging the parents through LDS as
 // well, as the other step kernels do, measured 1.13x slower when two waves fit.
 // kRows children a wavefront: see branch_rows().
@@ -1073,8 +1072,8 @@ __global__ __launch_bounds__(kPlayThreads) void branch_observe_kernel(
       for (int k = 0; k < kRowWords; ++k) out[k] = row[k];
     }
   }
-  // Keeping the child in registers through the observation costs the third wave a SIMD (204
-  // VGPRs against 173), but the rows written before it are slower where the output passes
+  // Keeping the child in registers through the observation costs the third wave a SIMD (200
+  // VGPRs), but the rows written before it are slower where the output passes
   // the last-level cache: 1,048,576 children 670 us so, 737 with the rows from registers
   // right after the step, 698 with wave 1 copying them from LDS beside the observation.
   store_observation<2, false, kRows>(t.out, base, count, features, legal, &next_item);  // wave 0 after its rows
