@@ -503,7 +503,7 @@ def canonical_workload(ext, torch, games: int = 131072, iters: int = 8) -> dict:
                          "traffic": measured_traffic("canonical_kernel", str(games)),
                          "bytes_per_game": 56, "avg_launch_ms": round(ms, 4),
                          "bound_note": "HBM is not what bounds it: VALU issue is (SQ counters: "
-                                       "VALU busy 0.67 at 131,072 games, 0.78 at 1,048,576)"}}
+                                       "VALU busy 0.70 at 131,072 games, 1.05 at 1,048,576)"}}
 
 
 def decode_lengths(torch, events: "torch.Tensor", slots: int, seed: int) -> dict:

@@ -24,8 +24,9 @@
 //   * LDS holds Z, the 128 x 512 bf16 input of the current layer (128 KiB), and U, one
 //     128-column chunk of relu(fc1) (32 KiB): fc1 and fc2 run chunk by chunk, fc1's chunk
 //     on a 2 x 4 grid of wavefronts (64 rows x 32 columns each) into U, then h += U W2's
-//     matching K slice.  Z and U store 16-byte group g of row r at g ^ (r & 7), so the 16
-//     rows of an A fragment read 8 different bank slots without padding (160 KiB in all);
+//     matching K slice.  Z and U are laid out K step by K step with a row's four 16-byte
+//     groups swizzled (swz), so an A fragment covers every bank without padding (160 KiB in
+//     all);
 //   * the input x passes through Z in two column slices ([0, 512) and [512, 768));
 //   * B fragments come from weights packed once in fragment order (cugo_mlp_pack_weight):
 //     the 64 lanes' 8 values of one (16-row tile, K step) are 1 KiB of contiguous memory,
