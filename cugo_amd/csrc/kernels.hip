@@ -799,7 +799,7 @@ void play_kernel(
 //   * wave 1 observes: it unpacks that row, builds the observation's records and stores
 //     them, one step behind (wave 0 takes over what is left of larger tiles' stores).
 // So the latency of a step is the longer of the two parts instead of their sum: 3,001 games
-// on 4-game tiles 413 -> 318 us a 32-step launch.  One barrier a step hands a state over;
+// on 4-game tiles 413 -> 305 us a 32-step launch.  One barrier a step hands a state over;
 // wave 0 overwrites the row in LDS only once wave 1 has counted it as unpacked (`seen`;
 // wave 1 unpacks first thing after the barrier, so wave 0 does not wait in practice).  An
 // action that fails reads its state again from that row.  At 65,536 games, where the
@@ -1453,7 +1453,8 @@ inline int device_cus() {
 // finishes first; once every SIMD has one or two, fewer games a tile only add wavefronts
 // that wait for a SIMD.  The lines lie where a grid passes one or two wavefronts a SIMD
 // (1,024 SIMDs).  Measured on MI355X, us a call (64 / 32 / 16 / 8 / 4 games a tile, graphs
-// or bursts of launches on mid-game rows; the start of a launch is ~3 us of each):
+// or bursts of launches on mid-game rows; the start of a launch is ~3 us of each; the kernels
+// have since become up to 5 % faster):
 //   play_random x 32    n = 3,001: 828 / 548 / 408 / 386 / 321     8,192: 808 / 552 / 460 / 374
 //                       16,384: 819 / 612 / 485                    32,768: 900 / 661
 //   observe             700: 19.6 / 14.3 / 11.4 / 9.6 / 8.5        4,096: 20.6 / 15.5 / 12.5 / 12.1 / 11.7
